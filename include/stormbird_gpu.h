@@ -268,6 +268,10 @@ int sb_debug_gauss_device(const double* A, const double* b, size_t n, double* x,
  * systems (16-column panels, trailing updates, one-wave back substitution), the
  * matrix in global memory: n <= 1024.  Returns as sb_debug_gauss_device. */
 int sb_debug_gauss_blocked_device(const double* A, const double* b, size_t n, double* x);
+/* The ordered sum that the fixed velocities' fold runs on one wave, on given terms:
+ * out[0] = (((s0 + terms[0]) + terms[1]) + ...), rounded after every addition
+ * (s0 not -0).  Returns 0, -1 on bad arguments, -2 on a device error. */
+int sb_debug_ordered_sum_device(const double* terms, size_t n, double s0, double* out);
 
 /* ---- Batched simulations ------------------------------------------------
  * Many independent simulations (each built from its own setup string, with

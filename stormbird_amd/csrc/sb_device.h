@@ -130,7 +130,7 @@ struct McBuffers {
 };
 
 // Scratch of the two-pass few-target sum (k_terms + k_fold_terms): one chunk
-// of per-pair terms [3][chunk][ld] and the running sums [3][n_targets].
+// of per-pair terms [3][n_targets][row] and the running sums [3][n_targets].
 struct FoldBuffers {
     double* terms = nullptr;
     long cap = 0;                 // doubles in `terms`
@@ -145,8 +145,13 @@ hipError_t launch_init_wake(const Inst& d, double dt, int use_mean_velocity, con
 hipError_t launch_wake_step(const Inst& d, double dt, hipStream_t st);
 hipError_t launch_panels(const Inst& d, const double* pts, int shift_strengths, hipStream_t st);
 // Fixed velocities at the control points (rows >= 1).  Two-pass sum when `fb`
-// holds room for at least one 64-panel chunk, else one wave per target.
+// holds room for at least one 1,024-panel chunk, else one wave per target.
 hipError_t launch_fixed(const Inst& d, int mode, FoldBuffers* fb, hipStream_t st);
+// Doubles of FoldBuffers::terms for n_panels panels: all of them, or the largest chunk
+// of at most 64 MiB (at least one 1,024-panel pass).
+long fold_terms_doubles(long n_targets, long n_panels);
+// out[0] = s0 plus terms[0..n) one after another (n a multiple of 1,024): the fold alone.
+hipError_t launch_ordered_sum(const double* terms, long n, double s0, double* out, hipStream_t st);
 hipError_t launch_factors(const Inst& d, hipStream_t st);
 // Quasi-steady factors: F[j][i] = unit velocity of strip j's horseshoe vortex at ctrl point i.
 hipError_t launch_horseshoe_factors(const Inst& d, hipStream_t st);

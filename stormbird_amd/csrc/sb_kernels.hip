@@ -975,101 +975,208 @@ __global__ __launch_bounds__(256) void k_fold(Inst d, const double* __restrict__
     if (t < n_targets && lane == 0) store3(out + 3 * t, acc);
 }
 
-// Few targets, many panels, in two passes over a chunk of panels
-// [p_begin, p_begin + cnt):
-//  k_terms      every (target, panel) term strength * u, one wave per 64
-//               targets x tp panels (tp <= 16: fewer when the chunk would give
-//               too few waves to fill the GPU), written to terms[c][q][t]
-//               (ld >= n_targets);
-//               a skipped panel (zero strength, or the target's own wing in
-//               neglect-self mode) writes +0;
-//  k_fold_terms one lane per (component, target) chain adds the chunk's terms
-//               in ascending panel order to the running sum acc[c][t] (fed
-//               through LDS by a whole workgroup of loaders).
-// Adding +0 leaves a sum unchanged unless the sum is -0, and a sum that starts
-// at +0 never becomes -0, so the result equals the reference's fold that
-// skips those panels (induced_velocity_calc.rs:111-150, 202-210).
-constexpr int TERM_PANELS = 16;
+__device__ inline double readlane_f64(double v, int lane) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
 
-template <int MODE>
-__global__ __launch_bounds__(256) void k_terms(Inst d, const double* __restrict__ targets, int n_targets,
-                                               long p_begin, long cnt, int neglect, double* __restrict__ terms,
-                                               int ld, int tp) {
-    int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    int t = blockIdx.y * WAVE + lane;
-    int tc = t < n_targets ? t : n_targets - 1;
-    V3 x = load3(targets + 3 * tc);
-    int wt = neglect ? d.wing_of[tc] : -1;
-    long q0 = ((long)blockIdx.x * 4 + wave) * tp;
-    for (int j = 0; j < tp; ++j) {
-        long q = q0 + j;
-        if (q >= cnt) break;
-        int k = __builtin_amdgcn_readfirstlane((int)(p_begin + q));
-        PanelRec r = d.rec[k];
-        V3 term{0.0, 0.0, 0.0};
-        bool skip = r.strength == 0.0 || (neglect && d.wing_of[k % d.N] == wt);
-        if (!skip) term = unit_velocity_sym<MODE>(d, r, k, x) * r.strength;
-        if (t < n_targets) {
-            terms[(0 * cnt + q) * ld + t] = term.x;
-            terms[(1 * cnt + q) * ld + t] = term.y;
-            terms[(2 * cnt + q) * ld + t] = term.z;
+// ---- ordered sums by speculation ----------------------------------------------
+// s = (((s + p_0) + p_1) + ...) over the 64 M terms of a wave (lane l holds terms
+// l M .. l M + M - 1), rounded after every addition as the one-lane loop rounds:
+// the same bits, without its chain of 64 M dependent additions (~11 ns each
+// when fed through LDS).  Every lane runs its M additions at once, from a guess
+// g of the sum before its terms (a parallel prefix sum, right up to a few ulps);
+// the guesses are corrected afterwards:
+//  * while all partial sums stay in one binade, they live on one grid of spacing
+//    u, and shifting the incoming sum by an even number of u shifts every rounded
+//    partial sum by exactly that amount (round to nearest even commutes with
+//    such a shift).  A second run from the neighbour g + u serves odd shifts, where
+//    ties round the other way.  So a lane maps an incoming offset d (in units of
+//    the last place, relative to g) to the outgoing offset relative to the next
+//    lane's guess, d + E[d & 1]; such maps compose associatively, and a scan
+//    over the lanes gives every lane's offset;
+//  * a lane whose partial sums (of either run), widened by 2^32 ulps, leave the
+//    binade, or whose offsets are not small, adds its terms once more from its
+//    exact incoming sum, and the scan restarts behind it.  Zero, subnormal,
+//    infinite and NaN sums take that way too.
+// All lanes get the result.  The sum must not be -0 on entry (a sum that starts at
+// +0 never is).  A pass of 1,024 terms takes ~1 us of one wave (16 terms per lane),
+// where the chain of additions took ~11; sums that change binade at every step (terms
+// that cancel to zero) fall back to about the chain's own time.
+template <int CTRL, int ROWS = 0xf>
+__device__ inline int dpp_i32(int old, int v) {
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS = 0xf>
+__device__ inline double dpp_add_f64(double v) {  // v + (v of the lane CTRL names; +0 where there is none)
+    const int lo = dpp_i32<CTRL, ROWS>(0, __double2loint(v)), hi = dpp_i32<CTRL, ROWS>(0, __double2hiint(v));
+    return v + __hiloint2double(hi, lo);
+}
+template <int CTRL, int ROWS = 0xf>
+__device__ inline void dpp_compose(int& e0, int& e1) {  // the map of the lane CTRL names, then this lane's
+    const int p0 = dpp_i32<CTRL, ROWS>(0, e0), p1 = dpp_i32<CTRL, ROWS>(0, e1);
+    const int n0 = p0 + ((p0 & 1) ? e1 : e0), n1 = p1 + ((p1 & 1) ? e0 : e1);
+    e0 = n0;
+    e1 = n1;
+}
+constexpr int DPP_ROW_SHR = 0x110, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138, DPP_BCAST15 = 0x142, DPP_BCAST31 = 0x143;
+
+template <int M>
+__device__ inline double ordered_sum_wave(double s, const double (&p)[M]) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    double own = p[0];
+    bool zero = p[0] == 0.0;
+#pragma unroll
+    for (int k = 1; k < M; ++k) {
+        own = own + p[k];
+        zero = zero & (p[k] == 0.0);
+    }
+    double inc = own;
+    inc = dpp_add_f64<DPP_ROW_SHR + 1>(inc);
+    inc = dpp_add_f64<DPP_ROW_SHR + 2>(inc);
+    inc = dpp_add_f64<DPP_ROW_SHR + 4>(inc);
+    inc = dpp_add_f64<DPP_ROW_SHR + 8>(inc);
+    inc = dpp_add_f64<DPP_BCAST15, 0xa>(inc);
+    inc = dpp_add_f64<DPP_BCAST31, 0xc>(inc);
+    const double g = s + __hiloint2double(dpp_i32<DPP_WAVE_SHR1>(0, __double2hiint(inc)),
+                                          dpp_i32<DPP_WAVE_SHR1>(0, __double2loint(inc)));
+    const long long gb = __double_as_longlong(g);
+    double a = g, b = __longlong_as_double(gb + 1);
+    unsigned hmin = (unsigned)__double2hiint(a), hmax = hmin;
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+        a = a + p[k];
+        b = b + p[k];
+        const unsigned ha = (unsigned)__double2hiint(a), hb = (unsigned)__double2hiint(b);
+        hmin = min(hmin, min(ha, hb));
+        hmax = max(hmax, max(ha, hb));
+    }
+    const long long ab = __double_as_longlong(a), bb = __double_as_longlong(b) - 1;
+    // the next lane's guess; lane 63 refers its result to its own run
+    const int nhi = dpp_i32<DPP_WAVE_SHL1>(__double2hiint(a), __double2hiint(g));
+    const int nlo = dpp_i32<DPP_WAVE_SHL1>(__double2loint(a), __double2loint(g));
+    const long long nb = __double_as_longlong(__hiloint2double(nhi, nlo));
+    hmin = min(hmin, (unsigned)nhi);
+    hmax = max(hmax, (unsigned)nhi);
+    const long long d0 = ab - nb, d1 = bb - nb;
+    constexpr long long SMALL = 1ll << 24;
+    const unsigned lo12 = (hmin - 1u) >> 20, hi12 = (hmax + 1u) >> 20, ex = lo12 & 0x7ffu;
+    bool fine = lo12 == hi12 && ex != 0u && ex != 0x7ffu;
+    fine = fine && d0 > -SMALL && d0 < SMALL && d1 > -SMALL && d1 < SMALL;
+    fine = fine || (zero && gb == nb);  // adding zeros changes nothing
+    const unsigned long long good = __ballot(fine);
+    const int f0 = fine ? (int)d0 : 0, f1 = fine ? (int)d1 : 0;
+    int j0 = 0;         // lanes below are done; sx is the exact sum before lane j0
+    double sx = s;
+    for (;;) {
+        const long long g0 = __double_as_longlong(readlane_f64(g, j0));
+        const long long o = __double_as_longlong(sx) - g0;
+        int j = j0;     // the next lane to add from its exact incoming sum
+        if (((good >> j0) & 1ull) && o > -SMALL && o < SMALL) {
+            int e0 = lane < j0 ? 0 : f0, e1 = lane < j0 ? 0 : f1;
+            dpp_compose<DPP_ROW_SHR + 1>(e0, e1);
+            dpp_compose<DPP_ROW_SHR + 2>(e0, e1);
+            dpp_compose<DPP_ROW_SHR + 4>(e0, e1);
+            dpp_compose<DPP_ROW_SHR + 8>(e0, e1);
+            dpp_compose<DPP_BCAST15, 0xa>(e0, e1);
+            dpp_compose<DPP_BCAST31, 0xc>(e0, e1);
+            const unsigned long long bad = ~good & (~0ull << j0);
+            const int last = bad ? (int)__builtin_ctzll(bad) - 1 : WAVE - 1;
+            const int d = (int)o + __builtin_amdgcn_readlane((o & 1) ? e1 : e0, last);
+            sx = __longlong_as_double(__double_as_longlong(readlane_f64(__longlong_as_double(nb), last)) + d);
+            if (!bad) return sx;
+            j = last + 1;
         }
+        double v = sx;
+#pragma unroll
+        for (int k = 0; k < M; ++k) v = v + p[k];
+        sx = readlane_f64(v, j);
+        j0 = j + 1;
+        if (j0 == WAVE) return sx;
     }
 }
 
-// One workgroup (16 waves) per 16 chains of one component: every thread keeps
-// FOLD_K loads of the next 512-row block in flight while lanes 0-15 of wave 0
-// add the current block (double-buffered in LDS) in ascending row order.
-constexpr int FOLD_CH = 16;
-constexpr int FOLD_K = 8;
-constexpr int FOLD_THREADS = 1024;
-constexpr int FOLD_ROWS = FOLD_THREADS * FOLD_K / FOLD_CH;  // 512
+// The 64 M terms at src in order, as ordered_sum_wave takes them (src 16-byte aligned).
+constexpr int SUM_M = 16;
+constexpr int SUM_ROWS = WAVE * SUM_M;  // terms per pass of a wave
+__device__ inline void load_terms(const double* src, double (&p)[SUM_M]) {
+    const double2* q = (const double2*)(src + (threadIdx.x & (WAVE - 1)) * SUM_M);
+#pragma unroll
+    for (int k = 0; k < SUM_M / 2; ++k) {
+        const double2 v = q[k];
+        p[2 * k] = v.x;
+        p[2 * k + 1] = v.y;
+    }
+}
+// s plus the `passes` x SUM_ROWS terms at src, in order; the next pass's terms are in
+// flight while a pass is summed.
+__device__ inline double ordered_sum(double s, const double* src, long passes) {
+    if (passes <= 0) return s;
+    double p[SUM_M], q[SUM_M];
+    load_terms(src, p);
+    for (long b = 0; b < passes; ++b) {
+        const long n = b + 1 < passes ? b + 1 : b;
+        load_terms(src + n * SUM_ROWS, q);
+        s = ordered_sum_wave<SUM_M>(s, p);
+#pragma unroll
+        for (int k = 0; k < SUM_M; ++k) p[k] = q[k];
+    }
+    return s;
+}
 
-__global__ __launch_bounds__(1024) void k_fold_terms(const double* __restrict__ terms, int ld, int n_targets,
-                                                     long cnt, int first, double* __restrict__ acc,
-                                                     double* __restrict__ out) {
-    __shared__ double buf[2][FOLD_ROWS][FOLD_CH];
-    const int groups = (n_targets + FOLD_CH - 1) / FOLD_CH;
-    const int c = blockIdx.x / groups;
-    const int t0 = (blockIdx.x % groups) * FOLD_CH;
-    const double* src = terms + (long)c * cnt * ld + t0;  // t0 + FOLD_CH <= ld: loads stay in the chunk
-    const int lc = threadIdx.x % FOLD_CH, r0 = threadIdx.x / FOLD_CH;
-    constexpr int RSTEP = FOLD_THREADS / FOLD_CH;  // 64
-    const long nb = (cnt + FOLD_ROWS - 1) / FOLD_ROWS;
-    double r[FOLD_K];
-    auto load = [&](long b) {
-#pragma unroll
-        for (int k = 0; k < FOLD_K; ++k) {
-            long q = b * FOLD_ROWS + r0 + RSTEP * k;
-            r[k] = q < cnt ? src[q * ld + lc] : 0.0;
-        }
-    };
-    auto store = [&](int slot) {
-#pragma unroll
-        for (int k = 0; k < FOLD_K; ++k) buf[slot][r0 + RSTEP * k][lc] = r[k];
-    };
-    const int t = t0 + (int)threadIdx.x;
-    const bool folder = threadIdx.x < FOLD_CH && t < n_targets;
-    double s = (folder && !first) ? acc[(long)c * n_targets + t] : 0.0;
-    if (nb > 0) {
-        load(0);
-        store(0);
+// Few targets, many panels, in two passes over a chunk of panels
+// [p_begin, p_begin + cnt):
+//  k_terms      every (target, panel) term strength * u, one panel per lane, `tg`
+//               targets per block row, written to terms[c][t][q] (row length ld,
+//               a multiple of SUM_ROWS); a skipped panel (zero strength, or the
+//               target's own wing in neglect-self mode) and the padding q >= cnt
+//               write +0;
+//  k_fold_terms one wave per (component, target) chain adds the chunk's terms
+//               in ascending panel order to the running sum acc[c][t].
+// Adding +0 leaves a sum unchanged unless the sum is -0, and a sum that starts
+// at +0 never becomes -0, so the result equals the reference's fold that
+// skips those panels (induced_velocity_calc.rs:111-150, 202-210).
+// A lane's panel record stays in registers for its targets, and the terms of a
+// chain are contiguous, as the fold reads them.  160 targets x 160,000 panels:
+// terms 0.32 -> 0.21 ms (FP64 issue), fold 1.77 -> 0.18 ms (the scan of every
+// pass); 20 x 3,980 panels: 11 -> 6.5 us and 42 -> 6.4 us (kernel times).
+template <int MODE>
+__global__ __launch_bounds__(256) void k_terms(Inst d, const double* __restrict__ targets, int n_targets,
+                                               long p_begin, long cnt, int neglect, double* __restrict__ terms,
+                                               long ld, int tg) {
+    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;  // q < ld: the grid covers a row exactly
+    const bool in = q < cnt;
+    const int k = (int)(p_begin + (in ? q : cnt - 1));
+    const PanelRec r = d.rec[k];
+    const int wk = neglect ? d.wing_of[k % d.N] : -1;
+    const int t0 = blockIdx.y * tg, t1 = t0 + tg < n_targets ? t0 + tg : n_targets;
+    for (int t = t0; t < t1; ++t) {
+        const V3 x = load3(targets + 3 * t);
+        V3 term{0.0, 0.0, 0.0};
+        const bool skip = !in || r.strength == 0.0 || (neglect && d.wing_of[t] == wk);
+        if (!skip) term = unit_velocity_sym<MODE>(d, r, k, x) * r.strength;
+        terms[((long)0 * n_targets + t) * ld + q] = term.x;
+        terms[((long)1 * n_targets + t) * ld + q] = term.y;
+        terms[((long)2 * n_targets + t) * ld + q] = term.z;
     }
-    __syncthreads();
-    for (long b = 0; b < nb; ++b) {
-        if (b + 1 < nb) load(b + 1);
-        if (folder) {
-            int rows = cnt - b * FOLD_ROWS < FOLD_ROWS ? (int)(cnt - b * FOLD_ROWS) : FOLD_ROWS;
-            const double(*cur)[FOLD_CH] = buf[b & 1];
-            for (int q = 0; q < rows; ++q) s = s + cur[q][threadIdx.x];
-        }
-        if (b + 1 < nb) store((int)((b + 1) & 1));
-        __syncthreads();
-    }
-    if (folder) {
-        acc[(long)c * n_targets + t] = s;
+}
+
+__global__ __launch_bounds__(64) void k_fold_terms(const double* __restrict__ terms, long ld, int n_targets, int first,
+                                                   double* __restrict__ acc, double* __restrict__ out) {
+    const int chain = blockIdx.x;  // component c of target t
+    const int c = chain / n_targets, t = chain - c * n_targets;
+    const double s = ordered_sum(first ? 0.0 : acc[chain], terms + (long)chain * ld, ld / SUM_ROWS);
+    if (threadIdx.x == 0) {
+        acc[chain] = s;
         if (out) out[3 * t + c] = s;
     }
+}
+
+// The ordered sum on given terms (checks of the sum itself): n a multiple of SUM_ROWS.
+__global__ __launch_bounds__(64) void k_ordered_sum(const double* terms, long n, double s0, double* out) {
+    const double s = ordered_sum(s0, terms, n / SUM_ROWS);
+    if (threadIdx.x == 0) out[0] = s;
 }
 
 // frozen_wake.rs:198-261: F[j][i] = unit velocity of first-row panel j at ctrl point i.
@@ -1790,11 +1897,6 @@ SB_HD inline LinrLayout linr_layout(int N) {
 template <int V>
 SB_HD inline long linr_shared_doubles(int N) { return linr_layout<V>(N).total; }
 
-__device__ inline double readlane_f64(double v, int lane) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-    return __hiloint2double(hi, lo);
-}
 template <int CTRL>
 __device__ inline double dpp_f64(double v) {
     const int lo = __builtin_amdgcn_update_dpp(__double2loint(v), __double2loint(v), CTRL, 0xf, 0xf, false);
@@ -3033,28 +3135,28 @@ hipError_t launch_fixed(const Inst& d, int mode, FoldBuffers* fb, hipStream_t st
     int p_end = d.N * d.nz_rows;
     if (p_end < p_begin) p_end = p_begin;
     const double* ctrl = d.geo + d.gl.ctrl;
-    const int ld = (d.N + WAVE - 1) / WAVE * WAVE;
-    const long chunk = fb && fb->cap_targets >= d.N ? fb->cap / (3L * ld) / (4 * TERM_PANELS) * (4 * TERM_PANELS) : 0;
+    const long chunk = fb && fb->cap_targets >= d.N ? fb->cap / (3L * d.N) / SUM_ROWS * SUM_ROWS : 0;
     if (chunk > 0 && p_end > p_begin) {
         int first = 1;
         for (long b = p_begin; b < p_end; b += chunk) {
-            long cnt = p_end - b < chunk ? p_end - b : chunk;
-            // panels per wave: 16, or fewer while the chunk gives less than ~16 waves per CU
-            int tp = TERM_PANELS;
-            while (tp > 1 && (cnt + tp - 1) / tp * (ld / WAVE) < 4096) tp >>= 1;
-            dim3 grid(blocks_for(cnt, 4 * tp), (unsigned)(ld / WAVE));
+            const long cnt = p_end - b < chunk ? p_end - b : chunk;
+            const long ld = (cnt + SUM_ROWS - 1) / SUM_ROWS * SUM_ROWS;
+            // targets per wave: as many as leave 16 waves per CU (a wave's record load serves them all)
+            int tg = 16;
+            while (tg > 1 && ld / WAVE * ((d.N + tg - 1) / tg) < 4096) tg >>= 1;
+            const dim3 grid((unsigned)(ld / 256), (unsigned)((d.N + tg - 1) / tg));
             if (mode == MODE_FAST)
                 hipLaunchKernelGGL(k_terms<MODE_FAST>, grid, dim3(256), 0, st, d, ctrl, d.N, b, cnt, d.neglect_self,
-                                   fb->terms, ld, tp);
+                                   fb->terms, ld, tg);
             else if (mode == MODE_FP32_KAHAN)
                 hipLaunchKernelGGL(k_terms<MODE_FP32_KAHAN>, grid, dim3(256), 0, st, d, ctrl, d.N, b, cnt,
-                                   d.neglect_self, fb->terms, ld, tp);
+                                   d.neglect_self, fb->terms, ld, tg);
             else
                 hipLaunchKernelGGL(k_terms<MODE_EXACT>, grid, dim3(256), 0, st, d, ctrl, d.N, b, cnt, d.neglect_self,
-                                   fb->terms, ld, tp);
-            bool last = b + cnt >= p_end;
-            hipLaunchKernelGGL(k_fold_terms, dim3(3 * ((d.N + FOLD_CH - 1) / FOLD_CH)), dim3(FOLD_THREADS), 0, st,
-                               fb->terms, ld, d.N, cnt, first, fb->acc, last ? d.fixed : nullptr);
+                                   fb->terms, ld, tg);
+            const bool last = b + cnt >= p_end;
+            hipLaunchKernelGGL(k_fold_terms, dim3(3 * d.N), dim3(WAVE), 0, st, fb->terms, ld, d.N, first, fb->acc,
+                               last ? d.fixed : nullptr);
             first = 0;
         }
         return hipGetLastError();
@@ -3069,6 +3171,17 @@ hipError_t launch_fixed(const Inst& d, int mode, FoldBuffers* fb, hipStream_t st
     else
         hipLaunchKernelGGL(k_fold<MODE_EXACT>, dim3(nb), dim3(256), 0, st, d, ctrl, d.N, p_begin, p_end,
                            d.neglect_self, d.fixed);
+    return hipGetLastError();
+}
+
+long fold_terms_doubles(long n_targets, long n_panels) {
+    const long rows = (n_panels + SUM_ROWS - 1) / SUM_ROWS * SUM_ROWS, fit = (8L << 20) / (3 * n_targets) / SUM_ROWS * SUM_ROWS;
+    return 3 * n_targets * (rows < fit ? rows : fit < SUM_ROWS ? SUM_ROWS : fit);
+}
+
+hipError_t launch_ordered_sum(const double* terms, long n, double s0, double* out, hipStream_t st) {
+    if (n % SUM_ROWS != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_ordered_sum, dim3(1), dim3(WAVE), 0, st, terms, n, s0, out);
     return hipGetLastError();
 }
 

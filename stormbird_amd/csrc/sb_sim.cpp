@@ -452,6 +452,25 @@ int sb_debug_gauss_blocked_device(const double* A, const double* b, size_t n, do
     return rc;
 }
 
+int sb_debug_ordered_sum_device(const double* terms, size_t n, double s0, double* out) {
+    if (!terms || !out || n < 1 || n > (1u << 28)) return -1;
+    double* d = nullptr;
+    int rc = 0;
+    try {
+        const size_t padded = (n + 1023) / 1024 * 1024;  // +0 past the end leaves the sum unchanged
+        d = dalloc<double>(padded + 1);
+        check(hipMemset(d, 0, sizeof(double) * (padded + 1)), "memset");
+        check(hipMemcpy(d, terms, sizeof(double) * n, hipMemcpyHostToDevice), "upload");
+        check(launch_ordered_sum(d, (long)padded, s0, d + padded, nullptr), "ordered sum");
+        check(hipMemcpy(out, d + padded, sizeof(double), hipMemcpyDeviceToHost), "download");
+    } catch (const std::exception& e) {
+        g_error = e.what();
+        rc = -2;
+    }
+    if (d) (void)hipFree(d);
+    return rc;
+}
+
 int sb_debug_libm_host(int fn, const double* x, const double* y, double* out, size_t n) {
     if (!x || !out || (fn == 4 && !y)) return -1;
     for (size_t i = 0; i < n; ++i) {
