@@ -2499,12 +2499,16 @@ __global__ __launch_bounds__(1024) void k_gauss_blocked_finish(Inst d, double* x
 // Forces (force_calculations.rs:322-548, forces_and_moments.rs:163-245,
 // flow_derivatives.rs:31-62), one workgroup
 // ---------------------------------------------------------------------------
+constexpr int FORCE_CHUNK = 64;
 __device__ inline void forces_body(const Inst& d, double dt) {
+    __shared__ double terms[36][FORCE_CHUNK + 1];  // rows start in different banks
+    __shared__ int wing_lo[1024], wing_hi[1024];   // strips of each wing
     int N = d.N, W = d.W;
     const double* geo = d.geo;
     double* o = d.out;
     int i = threadIdx.x;
     double count = d.scal[3];
+    V3 F[6];
     if (i < N) {
         double gamma = o[OutLayout::gamma(N) + i];
         double alpha = o[OutLayout::alpha(N) + i];
@@ -2527,7 +2531,6 @@ __device__ inline void forces_body(const Inst& d, double dt) {
         double llen = geo[d.gl.local_len + i];
         V3 rel_out = load3(geo + d.gl.rel_out + 3 * i);
         V3 rel_local = load3(geo + d.gl.rel_local + 3 * i);
-        V3 F[6];
         F[0] = len(vel) == 0.0 ? V3{0.0, 0.0, 0.0} : (cross(vel, rel_out) * gamma) * rho;
         F[1] = V3{0.0, 0.0, 0.0};
         if (!d.viscous_lift_in_circulation) {
@@ -2571,25 +2574,58 @@ __device__ inline void forces_body(const Inst& d, double dt) {
         store3(d.hist + 3 * i, load3(d.hist + 3 * (N + i)));
         store3(d.hist + 3 * (N + i), ug);
     }
-    __syncthreads();
-    for (int idx = i; idx < 6 * W; idx += blockDim.x) {
-        int k = idx / W, w = idx - k * W;
-        int a = -1, b = -1;
-        for (int q = 0; q < N; ++q) {
-            if (d.wing_of[q] == w) {
-                if (a < 0) a = q;
-                b = q + 1;
+    // Integrated forces and moments: per (kind, wing, component of force or moment) one
+    // sum over the wing's strips in order from +0.  The strips' terms go through shared
+    // memory FORCE_CHUNK strips at a time (a virtual strip's as +0, which changes no sum
+    // that starts at +0); a thread per sum adds them, so a strip costs an LDS read and an
+    // addition instead of the dependent global loads of its forces (3 x 340 strips: 193 ->
+    // 32 us, 3 x 40: 22.5 -> 8.6, 20: 12.4 -> 7.8).
+    const bool real = i < N && geo[d.gl.is_virtual + i] == 0.0;
+    const V3 arm = i < N ? load3(geo + d.gl.ctrl_out + 3 * i) : V3{0.0, 0.0, 0.0};
+    if (i < N) {
+        const int w = d.wing_of[i];
+        if (i == 0 || d.wing_of[i - 1] != w) wing_lo[w] = i;
+        if (i == N - 1 || d.wing_of[i + 1] != w) wing_hi[w] = i + 1;
+    }
+    const int sums = 36 * W, per = (sums + (int)blockDim.x - 1) / (int)blockDim.x;
+    for (int p = 0; p < per; ++p) {
+        const int idx = p * (int)blockDim.x + i;  // kind, then force (0-2) or moment (3-5) component, then wing
+        const int w = idx % W, row = idx / W;
+        double s = 0.0;
+        for (int q0 = 0; q0 < N; q0 += FORCE_CHUNK) {
+            __syncthreads();
+            if (i >= q0 && i < q0 + FORCE_CHUNK && i < N) {
+#pragma unroll
+                for (int k = 0; k < 6; ++k) {
+                    const V3 f = real ? F[k] : V3{0.0, 0.0, 0.0}, m = real ? cross(arm, F[k]) : f;
+                    terms[6 * k][i - q0] = f.x;
+                    terms[6 * k + 1][i - q0] = f.y;
+                    terms[6 * k + 2][i - q0] = f.z;
+                    terms[6 * k + 3][i - q0] = m.x;
+                    terms[6 * k + 4][i - q0] = m.y;
+                    terms[6 * k + 5][i - q0] = m.z;
+                }
+            }
+            __syncthreads();
+            if (idx < sums) {
+                const int lo = wing_lo[w] > q0 ? wing_lo[w] - q0 : 0;
+                const int hi = wing_hi[w] < q0 + FORCE_CHUNK ? wing_hi[w] - q0 : FORCE_CHUNK;
+                int q = lo;
+                for (; q + 8 <= hi; q += 8) {
+                    double v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = terms[row][q + u];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) s = s + v[u];
+                }
+                for (; q < hi; ++q) s = s + terms[row][q];
             }
         }
-        V3 fs{0.0, 0.0, 0.0}, ms{0.0, 0.0, 0.0};
-        for (int q = a; a >= 0 && q < b; ++q) {
-            if (geo[d.gl.is_virtual + q] != 0.0) continue;
-            V3 f = load3(o + OutLayout::sect(N) + 3 * ((long)k * N + q));
-            fs = fs + f;
-            ms = ms + cross(load3(geo + d.gl.ctrl_out + 3 * q), f);
+        if (idx < sums) {
+            const int k = row / 6, c = row % 6;
+            const long at = c < 3 ? OutLayout::integ_f(N) + c : OutLayout::integ_m(N, W) + c - 3;
+            o[at + 3 * ((long)k * W + w)] = s;
         }
-        store3(o + OutLayout::integ_f(N) + 3 * ((long)k * W + w), fs);
-        store3(o + OutLayout::integ_m(N, W) + 3 * ((long)k * W + w), ms);
     }
     if (i == 0) {
         d.scal[3] = count + 1.0;
