@@ -995,11 +995,11 @@ __device__ inline double readlane_f64(double v, int lane) {
 //    ties round the other way.  So a lane maps an incoming offset d (in units of
 //    the last place, relative to g) to the outgoing offset relative to the next
 //    lane's guess, d + E[d & 1]; such maps compose associatively, and a scan
-//    over the lanes gives every lane's offset;
-//  * a lane whose partial sums (of either run), widened by 2^32 ulps, leave the
-//    binade, or whose offsets are not small, adds its terms once more from its
-//    exact incoming sum, and the scan restarts behind it.  Zero, subnormal,
-//    infinite and NaN sums take that way too.
+//    over each run of such lanes gives every lane's offset;
+//  * a lane whose partial sums may leave the binade (|g| -+ the sum of its terms'
+//    magnitudes, widened by 2^32 ulps), or whose offsets are not small, adds its terms
+//    once more from its exact incoming sum, and the run behind it starts there.  Zero,
+//    subnormal, infinite and NaN sums take that way too.
 // All lanes get the result.  The sum must not be -0 on entry (a sum that starts at
 // +0 never is).  A pass of 1,024 terms takes ~1 us of one wave (16 terms per lane),
 // where the chain of additions took ~11; sums that change binade at every step (terms
@@ -1014,8 +1014,9 @@ __device__ inline double dpp_add_f64(double v) {  // v + (v of the lane CTRL nam
     return v + __hiloint2double(hi, lo);
 }
 template <int CTRL, int ROWS = 0xf>
-__device__ inline void dpp_compose(int& e0, int& e1) {  // the map of the lane CTRL names, then this lane's
-    const int p0 = dpp_i32<CTRL, ROWS>(0, e0), p1 = dpp_i32<CTRL, ROWS>(0, e1);
+__device__ inline void dpp_compose(int& e0, int& e1, bool join) {  // join: the map of the lane CTRL names, then this lane's
+    const int q0 = dpp_i32<CTRL, ROWS>(0, e0), q1 = dpp_i32<CTRL, ROWS>(0, e1);
+    const int p0 = join ? q0 : 0, p1 = join ? q1 : 0;
     const int n0 = p0 + ((p0 & 1) ? e1 : e0), n1 = p1 + ((p1 & 1) ? e0 : e1);
     e0 = n0;
     e1 = n1;
@@ -1025,12 +1026,11 @@ constexpr int DPP_ROW_SHR = 0x110, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138,
 template <int M>
 __device__ inline double ordered_sum_wave(double s, const double (&p)[M]) {
     const int lane = threadIdx.x & (WAVE - 1);
-    double own = p[0];
-    bool zero = p[0] == 0.0;
+    double own = p[0], reach = fabs(p[0]);
 #pragma unroll
     for (int k = 1; k < M; ++k) {
         own = own + p[k];
-        zero = zero & (p[k] == 0.0);
+        reach = reach + fabs(p[k]);
     }
     double inc = own;
     inc = dpp_add_f64<DPP_ROW_SHR + 1>(inc);
@@ -1043,57 +1043,65 @@ __device__ inline double ordered_sum_wave(double s, const double (&p)[M]) {
                                           dpp_i32<DPP_WAVE_SHR1>(0, __double2loint(inc)));
     const long long gb = __double_as_longlong(g);
     double a = g, b = __longlong_as_double(gb + 1);
-    unsigned hmin = (unsigned)__double2hiint(a), hmax = hmin;
 #pragma unroll
     for (int k = 0; k < M; ++k) {
         a = a + p[k];
         b = b + p[k];
-        const unsigned ha = (unsigned)__double2hiint(a), hb = (unsigned)__double2hiint(b);
-        hmin = min(hmin, min(ha, hb));
-        hmax = max(hmax, max(ha, hb));
     }
     const long long ab = __double_as_longlong(a), bb = __double_as_longlong(b) - 1;
     // the next lane's guess; lane 63 refers its result to its own run
     const int nhi = dpp_i32<DPP_WAVE_SHL1>(__double2hiint(a), __double2hiint(g));
     const int nlo = dpp_i32<DPP_WAVE_SHL1>(__double2loint(a), __double2loint(g));
     const long long nb = __double_as_longlong(__hiloint2double(nhi, nlo));
-    hmin = min(hmin, (unsigned)nhi);
-    hmax = max(hmax, (unsigned)nhi);
     const long long d0 = ab - nb, d1 = bb - nb;
     constexpr long long SMALL = 1ll << 24;
-    const unsigned lo12 = (hmin - 1u) >> 20, hi12 = (hmax + 1u) >> 20, ex = lo12 & 0x7ffu;
-    bool fine = lo12 == hi12 && ex != 0u && ex != 0x7ffu;
+    const unsigned lo12 = ((unsigned)__double2hiint(fabs(g) - reach) - 1u) >> 20;
+    const unsigned hi12 = ((unsigned)__double2hiint(fabs(g) + reach) + 1u) >> 20;
+    bool fine = lo12 == hi12 && hi12 != 0u && hi12 != 0x7ffu;  // |g| - reach < 0: its sign bit makes them differ
     fine = fine && d0 > -SMALL && d0 < SMALL && d1 > -SMALL && d1 < SMALL;
-    fine = fine || (zero && gb == nb);  // adding zeros changes nothing
+    fine = fine || (reach == 0.0 && gb == nb);  // adding zeros changes nothing
     const unsigned long long good = __ballot(fine);
-    const int f0 = fine ? (int)d0 : 0, f1 = fine ? (int)d1 : 0;
-    int j0 = 0;         // lanes below are done; sx is the exact sum before lane j0
+    // Lanes below j0 are done (leading lanes of zeros change nothing); sx is the exact
+    // sum before lane j0, which is the first of its run or follows leading zeros.
+    const unsigned long long some = __ballot(!(reach == 0.0));
+    if (!some) return s;
+    int j0 = (int)__builtin_ctzll(some);
     double sx = s;
+    unsigned long long bad = ~__ballot(fine);
     for (;;) {
-        const long long g0 = __double_as_longlong(readlane_f64(g, j0));
-        const long long o = __double_as_longlong(sx) - g0;
-        int j = j0;     // the next lane to add from its exact incoming sum
-        if (((good >> j0) & 1ull) && o > -SMALL && o < SMALL) {
-            int e0 = lane < j0 ? 0 : f0, e1 = lane < j0 ? 0 : f1;
-            dpp_compose<DPP_ROW_SHR + 1>(e0, e1);
-            dpp_compose<DPP_ROW_SHR + 2>(e0, e1);
-            dpp_compose<DPP_ROW_SHR + 4>(e0, e1);
-            dpp_compose<DPP_ROW_SHR + 8>(e0, e1);
-            dpp_compose<DPP_BCAST15, 0xa>(e0, e1);
-            dpp_compose<DPP_BCAST31, 0xc>(e0, e1);
-            const unsigned long long bad = ~good & (~0ull << j0);
-            const int last = bad ? (int)__builtin_ctzll(bad) - 1 : WAVE - 1;
-            const int d = (int)o + __builtin_amdgcn_readlane((o & 1) ? e1 : e0, last);
-            sx = __longlong_as_double(__double_as_longlong(readlane_f64(__longlong_as_double(nb), last)) + d);
-            if (!bad) return sx;
-            j = last + 1;
-        }
-        double v = sx;
+        // compositions over the run of fine lanes that ends with this lane, `run` lanes long
+        const unsigned long long upto = bad & (~0ull >> (WAVE - 1 - lane));
+        const int run = upto ? lane - (WAVE - 1 - (int)__builtin_clzll(upto)) : lane + 1;
+        int e0 = run ? (int)d0 : 0, e1 = run ? (int)d1 : 0;
+        dpp_compose<DPP_ROW_SHR + 1>(e0, e1, run > 1);
+        dpp_compose<DPP_ROW_SHR + 2>(e0, e1, run > 2);
+        dpp_compose<DPP_ROW_SHR + 4>(e0, e1, run > 4);
+        dpp_compose<DPP_ROW_SHR + 8>(e0, e1, run > 8);
+        dpp_compose<DPP_BCAST15, 0xa>(e0, e1, run > (lane & 15) + 1);
+        dpp_compose<DPP_BCAST31, 0xc>(e0, e1, run > (lane & 31) + 1);
+        bool far = false;
+        while (!far) {
+            int j = j0;  // the next lane to add from its exact incoming sum
+            if (!((bad >> j0) & 1ull)) {
+                const long long o = __double_as_longlong(sx) - __double_as_longlong(readlane_f64(g, j0));
+                far = o <= -SMALL || o >= SMALL;  // its guess is far off: a run of its own, the rest anew
+                if (!far) {
+                    const unsigned long long next = bad & (~0ull << j0);
+                    const int last = next ? (int)__builtin_ctzll(next) - 1 : WAVE - 1;
+                    const int d = (int)o + __builtin_amdgcn_readlane((o & 1) ? e1 : e0, last);
+                    sx = __longlong_as_double(__double_as_longlong(readlane_f64(__longlong_as_double(nb), last)) + d);
+                    if (!next) return sx;
+                    j = last + 1;
+                }
+            }
+            double v = sx;
 #pragma unroll
-        for (int k = 0; k < M; ++k) v = v + p[k];
-        sx = readlane_f64(v, j);
-        j0 = j + 1;
-        if (j0 == WAVE) return sx;
+            for (int k = 0; k < M; ++k) v = v + p[k];
+            sx = readlane_f64(v, j);
+            j0 = j + 1;
+            if (j0 == WAVE) return sx;
+        }
+        bad |= 1ull << (j0 - 1);
     }
 }
 
@@ -1701,109 +1709,120 @@ __device__ inline double lin_entry(const Inst& d, const LinRow& q, int r, int c)
 }
 
 
-// linalg.rs:92-101 by one wave over the factored matrix in global memory (A
-// column-major [N + 1][N]: a[i][j] = A[j N + i], column N the right-hand side),
-// N <= 1024.  Every lane runs the same ordered sum
-// sum = ((0 + a[i][i+1] x[i+1]) + a[i][i+2] x[i+2]) + ..., reading the products
-// a[i][j] x[j], j >= i + 2, from shared memory in groups of 16 (pb, two rows of
-// pstride >= N + 64; x in shared memory too): lane t forms the products of row
-// i - 1 while row i is summed, from matrix entries loaded one row earlier, every
-// slot from a valid index and +0.0 past the row's end (the sum starts at +0.0 and
-// cannot become -0.0).
-__device__ inline void back_substitute_wave_cm(const double* A, int N, double* x, double* pb, int pstride) {
-    constexpr int PS = 16;  // product slots per lane: rows of up to 1024 products
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int nsl = (N + WAVE - 1) / WAVE;  // slots in use
-    const long n = N;
-    double xprev = (A[n * n + N - 1] - 0.0) / A[(n - 1) * n + N - 1];
-    x[N - 1] = xprev;
-    double cu[PS];  // a[i-1][i+1+t] for the products formed at step i
+// linalg.rs:92-101 over the factored matrix in global memory (A column-major
+// [N + 1][N]: a[i][j] = A[j N + i], column N the right-hand side), N <= 64 M, by a
+// whole workgroup.  Row i needs sum = ((0 + a[i][i+1] x[i+1]) + a[i][i+2] x[i+2]) + ...
+// and every row the one below it, so the rows stay a chain; wave 0 runs it, each
+// row's sum by speculation (ordered_sum_wave: lane l holds columns l M .. l M + M - 1
+// and their unknowns; +0 in the columns <= i leaves a sum that starts at +0
+// unchanged).  The other waves bring the next 8 rows from memory to shared memory
+// (64-byte pieces of the columns) while 8 rows are summed.
+// 1,020 rows: 1.15 ms, 2,700 cycles a row (was 3.9 ms: one chain of dependent additions
+// on every lane, ~9 ns each).
+constexpr int BSUB_ROWS = 8;
+constexpr int BSUB_THREADS = 512;  // wave 0 may hold 256 registers: the next row's entries are read early
+template <int M>
+SB_HD inline int bsub_stride() { return WAVE * (M + 1) + 8; }  // doubles per row: lanes and rows start in different banks
+template <int M>
+SB_HD inline long bsub_doubles() { return 2L * BSUB_ROWS * bsub_stride<M>() + 4 * BSUB_ROWS; }  // two blocks of rows, their diagonals and right-hand sides
+template <int M>
+__device__ inline void back_substitute_group(const double* A, int N, double* x, double* sh) {
+    const int t = threadIdx.x, lane = t & (WAVE - 1), stride = bsub_stride<M>();
+    double* diag = sh + 2L * BSUB_ROWS * stride;
+    double* rhs = diag + 2 * BSUB_ROWS;
+    for (int q = t; q < 2 * BSUB_ROWS * stride; q += (int)blockDim.x) sh[q] = 0.0;  // the columns <= i stay +0
+    __syncthreads();
+    // rows 8 q .. 8 q + 7 into the buffer of q's parity, every load of a thread in flight at once
+    auto load = [&](int q, int first, int threads) {
+        double* buf = sh + (long)(q & 1) * BSUB_ROWS * stride;
+        const int i0 = q * BSUB_ROWS, cnt = (N + 1 - i0) * BSUB_ROWS;
+        constexpr int PER = 19;  // 448 threads: 8 x 1,025 entries
+        for (int e0 = t - first; e0 < cnt; e0 += PER * threads) {
+            double v[PER];
 #pragma unroll
-    for (int s = 0; s < PS; ++s) {
-        const int r = N >= 3 ? N - 3 : 0;
-        cu[s] = s < nsl ? A[(long)min(N - 1 + lane + WAVE * s, N - 1) * n + r] : 0.0;
-    }
-    for (int i = N - 2; i >= 0; --i) {
-        const double di = A[(long)i * n + i], bi = A[n * n + i], u1 = A[(long)(i + 1) * n + i];
-        double nu[PS];  // a[i-2][i+t], t < N - i: the products formed at step i - 1
-        const int r2 = i >= 2 ? i - 2 : 0;
+            for (int u = 0; u < PER; ++u) {
+                const int e = min(e0 + u * threads, cnt - 1);
+                v[u] = A[(long)(i0 + e / BSUB_ROWS) * N + min(i0 + (e & (BSUB_ROWS - 1)), N - 1)];
+            }
 #pragma unroll
-        for (int s = 0; s < PS; ++s) nu[s] = s < nsl ? A[(long)min(i + lane + WAVE * s, N - 1) * n + r2] : 0.0;
-        const int lenp = i >= 1 ? N - i - 1 : 0;
-        double sum = 0.0 + u1 * xprev;
-        const int len = N - i - 2;
-        if (len > 0) {
-            const double2* p2 = (const double2*)(pb + (long)(i & 1) * pstride);
-            double2 c0 = p2[0], c1 = p2[1], c2 = p2[2], c3 = p2[3];
-            for (int g = 0; g < len; g += 16) {
-                const double2* nx = p2 + (g >> 1);
-                const double2 n0 = nx[4], n1 = nx[5], n2 = nx[6], n3 = nx[7];
-                sum += c0.x;
-                sum += c0.y;
-                sum += c1.x;
-                sum += c1.y;
-                sum += c2.x;
-                sum += c2.y;
-                sum += c3.x;
-                sum += c3.y;
-                c0 = nx[8];
-                c1 = nx[9];
-                c2 = nx[10];
-                c3 = nx[11];
-                sum += n0.x;
-                sum += n0.y;
-                sum += n1.x;
-                sum += n1.y;
-                sum += n2.x;
-                sum += n2.y;
-                sum += n3.x;
-                sum += n3.y;
+            for (int u = 0; u < PER; ++u) {
+                const int e = e0 + u * threads;
+                const int r = e & (BSUB_ROWS - 1), j = i0 + e / BSUB_ROWS, i = i0 + r;
+                if (e >= cnt || i >= N) continue;
+                if (j == N) rhs[(q & 1) * BSUB_ROWS + r] = v[u];
+                else if (j == i) diag[(q & 1) * BSUB_ROWS + r] = v[u];
+                else if (j > i) buf[r * stride + (j / M) * (M + 1) + j % M] = v[u];
             }
         }
-        double* po = pb + (long)((i - 1) & 1) * pstride;
+    };
+    // An even block's buffer next holds the even block two below it, whose columns
+    // <= i of this block's rows were never written: they lie left of what is loaded.
+    const int nq = (N + BSUB_ROWS - 1) / BSUB_ROWS;
+    load(nq - 1, 0, (int)blockDim.x);
+    __syncthreads();
+    double xr[M], a[M];  // the unknowns of the lane's columns, the current row's entries
 #pragma unroll
-        for (int s = 0; s < PS; ++s) {
-            if (s < nsl) {
-                const int t = lane + WAVE * s;
-                const double p = cu[s] * x[min(i + 1 + t, N - 1)];
-                po[t] = t < lenp ? p : 0.0;
+    for (int k = 0; k < M; ++k) xr[k] = 0.0;
+    for (int q = nq - 1; q >= 0; --q) {
+        if (t >= WAVE) {
+            if (q > 0) load(q - 1, WAVE, (int)blockDim.x - WAVE);
+        } else {
+            const double* buf = sh + (long)(q & 1) * BSUB_ROWS * stride;
+#pragma unroll
+            for (int r = BSUB_ROWS - 1; r >= 0; --r) {
+                const int i = q * BSUB_ROWS + r;
+                if (i >= N) continue;
+                const double* row = buf + r * stride + lane * (M + 1);
+                if (r == BSUB_ROWS - 1 || i == N - 1) {
+#pragma unroll
+                    for (int k = 0; k < M; ++k) a[k] = row[k];
+                }
+                double p[M];
+#pragma unroll
+                for (int k = 0; k < M; ++k) p[k] = a[k] * xr[k];
+                if (r > 0) {  // the next row's entries, under this row's sum
+#pragma unroll
+                    for (int k = 0; k < M; ++k) a[k] = row[k - stride];
+                }
+                const double bi = rhs[(q & 1) * BSUB_ROWS + r], di = diag[(q & 1) * BSUB_ROWS + r];
+                const double sum = ordered_sum_wave<M>(0.0, p);
+                const double xi = (bi - sum) / di;
+                if (lane == i / M) {
+                    x[i] = xi;
+                    if constexpr (M == 16) {  // i % 16 = r or r + 8
+                        if (q & 1) xr[8 + r] = xi;
+                        else xr[r] = xi;
+                    } else {
+                        xr[r % M] = xi;
+                    }
+                }
             }
         }
-        xprev = (bi - sum) / di;
-        x[i] = xprev;
-#pragma unroll
-        for (int s = 0; s < PS; ++s) cu[s] = nu[s];
+        __syncthreads();
     }
 }
 
 // Everything after the linear solve (linearized.rs:141-221): induced velocity,
 // viscous correction of the circulation, induced velocity again, residual and
-// outputs.  G holds the solution; R is [N] shared scratch.
-__device__ inline void lin_finish(const Inst& d, const Strip& s, double* G, double* R, int as_start) {
-    const int N = d.N;
-    const int t = threadIdx.x;
+// outputs.  In three parts, so that the blocked form can put the induced velocities
+// between them on the whole GPU.
+__device__ inline V3 lin_velocity(const Inst& d, const Strip& s, V3 ind, int as_start) {
+    return corrected_velocity(as_start ? 0 : d.vc_mode, d.vc_ratio, s.felt, ind);
+}
+SB_HD inline int lin_viscous(const Inst& d, int as_start) { return as_start ? 1 : !d.lin_disable_viscous; }
+SB_HD inline int lin_second_velocity(const Inst& d, int as_start) { return as_start ? 1 : d.lin_ivc; }
+// linearized.rs:156-197: the circulation corrected for the viscous lift at velocity u
+__device__ inline double lin_viscous_gamma(const Strip& s, double g, V3 u) {
+    const double a = angle_of_attack(s, u);
+    const double clf = foil_cl_pre_dropoff(*s.foil, a);
+    const double cll = foil_cl_linear(*s.foil, a);
+    return fabs(cll) > MIN_POSITIVE ? g * (clf / cll) : g;
+}
+// Strip t's outputs from its circulation and induced velocity; R is [N] shared scratch.
+__device__ inline void lin_outputs(const Inst& d, const Strip& s, double g, V3 u, double* R, int as_start) {
+    const int N = d.N, t = threadIdx.x;
     const bool act = t < N;
-    const int ic = act ? t : N - 1;
-    const int vc = as_start ? 0 : d.vc_mode;
-    const double vc_ratio = d.vc_ratio;
-    const int viscous = as_start ? 1 : !d.lin_disable_viscous;
-    const int ivc = as_start ? 1 : d.lin_ivc;
-    double g = G[ic];
-    const V3 ind1 = induced_at(d, s.fixed, G, ic);
-    V3 u = corrected_velocity(vc, vc_ratio, s.felt, ind1);
-    double a;
-    if (viscous) {  // linearized.rs:156-197
-        a = angle_of_attack(s, u);
-        double clf = foil_cl_pre_dropoff(*s.foil, a);
-        double cll = foil_cl_linear(*s.foil, a);
-        if (fabs(cll) > MIN_POSITIVE) g *= clf / cll;
-        __syncthreads();
-        if (act) G[t] = g;
-        __syncthreads();
-        // NoCorrection keeps the induced velocity of the linear solution
-        u = corrected_velocity(vc, vc_ratio, s.felt, ivc ? induced_at(d, s.fixed, G, ic) : ind1);
-    }
-    a = angle_of_attack(s, u);
+    const double a = angle_of_attack(s, u);
     if (as_start) {
         if (act) d.lin_gamma[t] = g;
         return;
@@ -1828,6 +1847,24 @@ __device__ inline void lin_finish(const Inst& d, const Strip& s, double* G, doub
         d.out[OutLayout::iters(N, d.W)] = 1.0;
         d.out[OutLayout::residual(N, d.W)] = sum / (double)N;
     }
+}
+// The one-workgroup form: G holds the solution.
+__device__ inline void lin_finish(const Inst& d, const Strip& s, double* G, double* R, int as_start) {
+    const int t = threadIdx.x;
+    const bool act = t < d.N;
+    const int ic = act ? t : d.N - 1;
+    double g = G[ic];
+    const V3 ind1 = induced_at(d, s.fixed, G, ic);
+    V3 u = lin_velocity(d, s, ind1, as_start);
+    if (lin_viscous(d, as_start)) {
+        g = lin_viscous_gamma(s, g, u);
+        __syncthreads();
+        if (act) G[t] = g;
+        __syncthreads();
+        // NoCorrection keeps the induced velocity of the linear solution
+        u = lin_velocity(d, s, lin_second_velocity(d, as_start) ? induced_at(d, s.fixed, G, ic) : ind1, as_start);
+    }
+    lin_outputs(d, s, g, u, R, as_start);
 }
 
 // ---- one-workgroup form (small N) -------------------------------------------
@@ -2231,9 +2268,12 @@ __global__ __launch_bounds__(LinrV<V>::T) void k_gauss_dense(const double* A, co
 }
 
 // ---- blocked form (matrix in global memory, d.lin) -------------------------
-// d.lin: [N + 1][N] matrix, then [N][8] row data (LinRow), then [N] ints: the
-// source position of every row after the current panel's exchanges.
+// d.lin: [N + 1][N] matrix, then [N][8] row data (LinRow; from the back substitution
+// on: the circulations [N] and induced velocities [N][3]), then [N] ints: the source position of every row after the
+// current panel's exchanges.
 __device__ inline double* lin_rows(const Inst& d) { return d.lin + (long)d.N * (d.N + 1); }
+__host__ __device__ inline double* lin_solution(const Inst& d) { return d.lin + (long)d.N * (d.N + 1); }
+__device__ inline double* lin_induced(const Inst& d) { return lin_solution(d) + d.N; }
 __device__ inline int* lin_perm(const Inst& d) { return (int*)(lin_rows(d) + 8L * d.N); }
 
 __global__ void k_lin_rows(Inst d) {
@@ -2265,85 +2305,108 @@ __global__ void k_lin_assemble(Inst d) {
     d.lin[idx] = c < N ? lin_entry(d, q, r, c) : -q.cll;
 }
 
-// Panel factorization of columns [k0, k0 + b), b <= 16: one workgroup of
-// LINP_T threads, thread t holding rows k0 + t + LINP_T s (s < 4) of the panel in
-// registers.  Rows are not exchanged while the panel is factored: every row keeps
-// its logical position.  Per pivot, each wave reduces its rows (the largest
-// magnitude, NaN excluded, ties to the lower position) and its best row publishes
-// its entries with the wave's result (LINP_SLOT doubles per wave, two sets by step
-// parity), and the row at position kk publishes its entries too (the pivot when it
-// holds NaN: linalg.rs:58-64 never replaces a NaN at the pivot position); after
-// one barrier every wave reduces the wave results and takes the pivot row from its
-// slot.  The factors replace the entries below the diagonal; rows are written back
-// at their logical positions, and the source position of every row goes to
-// lin_perm for the trailing update.
-constexpr int LINP_T = 256;                // threads of the panel kernel (4 rows each, N <= 1024)
-constexpr int LINP_W = LINP_T / 64;        // its waves
-constexpr int LINP_R = 4;                  // rows per thread
+// Panel factorization of columns [k0, k0 + b), b <= 16: one workgroup, thread t
+// holding row k0 + t of the panel in registers (a wave per 64 rows left).  Rows are
+// not exchanged while the panel is factored: every row keeps its logical position.
+// Per pivot, each wave reduces its rows (the largest magnitude, NaN excluded, ties
+// to the lower position) and its best row publishes its entries with the wave's
+// result (LINP_SLOT doubles per wave, two sets by step parity), and the row at
+// position kk publishes its entries too (the pivot when it holds NaN:
+// linalg.rs:58-64 never replaces a NaN at the pivot position); after one barrier
+// every wave reduces the wave results and takes the pivot row from its slot.  The
+// factors replace the entries below the diagonal; rows are written back at their
+// logical positions, and the source position of every row goes to lin_perm for the
+// trailing update.  A pivot is a chain of reductions, LDS round trips, a division and
+// a barrier, and every wave issues the reductions: with more waves than two per SIMD
+// they queue for issue, with four rows on each of 256 threads the rows' own work does
+// (1,020 rows, 64 panels: 1.45 ms; 1.52 with 16 waves, 2.6 with four rows).
+constexpr int LINP_W = 8;                  // waves of the panel kernel at most
+constexpr int LINP_T = LINP_W * WAVE;      // its threads; two rows each above LINP_T rows (N <= 1024)
 constexpr int LINP_SLOT = 20;              // a candidate row (16 entries), |v|, key, row at position kk, NaN flag
+template <int R>
 struct LinPanelState {
-    double a[LINP_R][16];
-    int pos[LINP_R];  // logical position of each row in the panel
-    bool done[LINP_R];
+    double a[R][16];
+    int pos[R];    // logical position of each row in the panel
+    bool done[R];  // a pivot already, or past the matrix
 };
+// The lane of the largest v >= 0 (NaN and negative values never win), ties to the
+// smallest key; -1 when no lane has one.  The high words are reduced first: one
+// 32-bit instruction per level, and they alone usually name the lane.
+__device__ inline int wave_argmax(double v, int key) {
+    const bool in = v >= 0.0;
+    const unsigned h = in ? (unsigned)__double2hiint(v) + 1u : 0u;
+    unsigned m = h;
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 1>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 2>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 4>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 8>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_BCAST15, 0xa>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_BCAST31, 0xc>(0, (int)m));
+    m = (unsigned)__builtin_amdgcn_readlane((int)m, WAVE - 1);
+    if (m == 0u) return -1;
+    unsigned long long top = __ballot(h == m);
+    if (top & (top - 1)) {
+        const bool cand = h == m;
+        const double best = wave_max_f64(cand ? v : -1.0);
+        const int k = wave_min_i32(cand && v == best ? key : 0x7fffffff);
+        top = __ballot(cand && v == best && key == k);
+    }
+    return (int)__builtin_ctzll(top);
+}
 // Pivot KK of the panel (a template, so that every register index is fixed).
 // Returns false at a singular pivot (recorded in scal[4]).
-template <int KK>
-__device__ __forceinline__ bool lin_panel_step(const Inst& d, int k0, int b, double* slots, double* pks, LinPanelState& st) {
-    constexpr int R = LINP_R;
+template <int KK, int R>
+__device__ __forceinline__ bool lin_panel_step(const Inst& d, int k0, double* slots, double* pks, LinPanelState<R>& st) {
     const int t = threadIdx.x, lane = t & (WAVE - 1), w = t >> 6;
-    double m = -1.0;
-#pragma unroll
-    for (int s = 0; s < R; ++s) m = fmax(m, st.done[s] ? -1.0 : fabs(st.a[s][KK]));  // NaN |v| never wins
-    const double Mw = wave_max_f64(m);
-    int key = 0x7fffffff;
+    double v = -1.0;
+    int key = 0x7fffffff;  // logical position * 1024 + row
+    bool second = false;   // the thread's candidate is its second row
 #pragma unroll
     for (int s = 0; s < R; ++s) {
-        const int kk2 = st.pos[s] * 1024 + t + LINP_T * s;
-        if (!st.done[s] && fabs(st.a[s][KK]) == Mw && kk2 < key) key = kk2;
+        const double vs = fabs(st.a[s][KK]);
+        const int ks = st.pos[s] * 1024 + t + LINP_T * s;
+        const bool take = !st.done[s] && (vs > v || (vs == v && ks < key));  // NaN never is
+        v = take ? vs : v;
+        key = take ? ks : key;
+        if (s > 0) second = take;
     }
-    const int Kw = wave_min_i32(key);
+    const int win = wave_argmax(v, key);
     double* sl = slots + ((KK & 1) * LINP_W + w) * LINP_SLOT;
     double* pk = pks + (KK & 1) * LINP_SLOT;
-    if (lane == 0) {
-        sl[16] = Mw;
-        sl[17] = (double)Kw;
+    if (lane == (win < 0 ? 0 : win)) {
+#pragma unroll
+        for (int c = KK; c < 16; ++c) sl[c] = R > 1 && second ? st.a[R - 1][c] : st.a[0][c];
+        sl[16] = win < 0 ? -1.0 : v;
+        sl[17] = (double)key;
     }
 #pragma unroll
     for (int s = 0; s < R; ++s) {
-        const int r = t + LINP_T * s;
-        if (Kw != 0x7fffffff && r == (Kw & 1023)) {
-#pragma unroll
-            for (int c = KK; c < 16; ++c)
-                if (c < b) sl[c] = st.a[s][c];
-        }
         if (!st.done[s] && st.pos[s] == KK) {
 #pragma unroll
-            for (int c = KK; c < 16; ++c)
-                if (c < b) pk[c] = st.a[s][c];
-            pk[16] = (double)r;
+            for (int c = KK; c < 16; ++c) pk[c] = st.a[s][c];
+            pk[16] = (double)(t + LINP_T * s);
             pk[17] = st.a[s][KK] != st.a[s][KK] ? 1.0 : 0.0;
         }
     }
     __syncthreads();
     double mr = -1.0;
     int kr = 0x7fffffff;
-    if (lane < LINP_W) {
+    if (lane < (int)blockDim.x / WAVE) {
         mr = slots[((KK & 1) * LINP_W + lane) * LINP_SLOT + 16];
         kr = (int)slots[((KK & 1) * LINP_W + lane) * LINP_SLOT + 17];
     }
-    const double M = wave_max_f64(mr);
-    const int K = wave_min_i32(mr == M ? kr : 0x7fffffff);
+    const int ww = wave_argmax(mr, kr);
     int pr, ppos;
     const double* prow;
-    if (pk[17] != 0.0) {  // NaN at the pivot position: that row
+    if (pk[17] != 0.0 || ww < 0) {  // NaN at the pivot position (as where every candidate is NaN): that row
         pr = (int)pk[16];
         ppos = KK;
         prow = pk;
     } else {
+        const int K = __builtin_amdgcn_readlane(kr, ww);
         pr = K & 1023;
         ppos = K >> 10;
-        prow = slots + ((KK & 1) * LINP_W + ((pr % LINP_T) >> 6)) * LINP_SLOT;
+        prow = slots + ((KK & 1) * LINP_W + ww) * LINP_SLOT;
     }
     const double piv = prow[KK];
     if (fabs(piv) < 1e-12) {  // uniform: every thread read the same slots
@@ -2352,8 +2415,7 @@ __device__ __forceinline__ bool lin_panel_step(const Inst& d, int k0, int b, dou
     }
 #pragma unroll
     for (int s = 0; s < R; ++s) {
-        const int r = t + LINP_T * s;
-        if (r == pr) {
+        if (t + LINP_T * s == pr) {
             st.pos[s] = KK;
             st.done[s] = true;
         } else if (!st.done[s] && st.pos[s] == KK) {
@@ -2362,45 +2424,42 @@ __device__ __forceinline__ bool lin_panel_step(const Inst& d, int k0, int b, dou
         if (!st.done[s]) {
             const double f = st.a[s][KK] / piv;
 #pragma unroll
-            for (int c = KK + 1; c < 16; ++c)
-                if (c < b) st.a[s][c] = st.a[s][c] - f * prow[c];
+            for (int c = KK + 1; c < 16; ++c) st.a[s][c] = st.a[s][c] - f * prow[c];
             st.a[s][KK] = f;
         }
     }
     return true;
 }
-template <int KK>
-struct LinPanelSteps {
-    __device__ __forceinline__ static bool run(const Inst& d, int k0, int b, double* slots, double* pks, LinPanelState& st) {
+template <int KK, int R>
+__device__ __forceinline__ bool lin_panel_steps(const Inst& d, int k0, int b, double* slots, double* pks, LinPanelState<R>& st) {
+    if constexpr (KK < 16) {
         if (KK >= b) return true;
-        if (!lin_panel_step<KK>(d, k0, b, slots, pks, st)) return false;
-        return LinPanelSteps<KK + 1>::run(d, k0, b, slots, pks, st);
+        if (!lin_panel_step<KK, R>(d, k0, slots, pks, st)) return false;
+        return lin_panel_steps<KK + 1, R>(d, k0, b, slots, pks, st);
     }
-};
-template <>
-struct LinPanelSteps<16> {
-    __device__ __forceinline__ static bool run(const Inst&, int, int, double*, double*, LinPanelState&) { return true; }
-};
+    return true;
+}
 
+template <int R>
 __global__ __launch_bounds__(LINP_T) void k_lin_panel(Inst d, int k0, int b) {
-    extern __shared__ double sh[];
-    if (d.scal[4] != 0.0) return;
+    __shared__ double slots[2 * LINP_W * LINP_SLOT];
+    __shared__ double pks[2 * LINP_SLOT];  // the row at position kk
+    const double singular = d.scal[4];  // read beside the panel, looked at after it
     const int N = d.N, t = threadIdx.x;
     const int nr = N - k0;
-    double* slots = sh;                              // [2][LINP_W][LINP_SLOT]
-    double* pks = slots + 2 * LINP_W * LINP_SLOT;    // [2][LINP_SLOT]: the row at position kk
-    LinPanelState st;
+    LinPanelState<R> st;
 #pragma unroll
-    for (int s = 0; s < LINP_R; ++s) {
+    for (int s = 0; s < R; ++s) {
         const int r = t + LINP_T * s;
         st.pos[s] = r;
         st.done[s] = r >= nr;  // past the panel: never a candidate, never updated
 #pragma unroll
         for (int c = 0; c < 16; ++c) st.a[s][c] = r < nr && c < b ? d.lin[(long)(k0 + c) * N + k0 + r] : 0.0;
     }
-    if (!LinPanelSteps<0>::run(d, k0, b, slots, pks, st)) return;
+    if (singular != 0.0) return;
+    if (!lin_panel_steps<0, R>(d, k0, b, slots, pks, st)) return;
 #pragma unroll
-    for (int s = 0; s < LINP_R; ++s) {
+    for (int s = 0; s < R; ++s) {
         const int r = t + LINP_T * s;
         if (r < nr) {
 #pragma unroll
@@ -2411,89 +2470,160 @@ __global__ __launch_bounds__(LINP_T) void k_lin_panel(Inst d, int k0, int b) {
     }
 }
 
-// Trailing update after the panel [k0, k0 + b): one workgroup per column j >=
-// k0 + b (the right-hand side included).  The panel's exchanges are applied as
-// one gather; the panel rows' entries take their updates from the earlier
-// pivots in order (these are the pivot rows' values), then every lower entry
-// takes the b updates a - l*u in pivot order.
+// Trailing update after the panel [k0, k0 + b): one workgroup per LIN_TRAIL_COLS
+// columns j >= k0 + b (the right-hand side included).  The panel's exchanges are
+// applied as one gather; the panel rows' entries take their updates from the earlier
+// pivots in order (these are the pivot rows' values: a lane per row, the finished
+// entry handed on by readlane), then every lower entry takes the b updates a - l*u in
+// pivot order.  A factor read serves the workgroup's columns (with one column per
+// workgroup the factors are read N times from the cache, and one thread for the panel
+// rows chained 120 dependent updates through memory: 1,020 rows, 64 launches: 1.34 ->
+// 0.59 ms).
 constexpr int LIN_TRAIL_THREADS = 256;
+constexpr int LIN_TRAIL_COLS = 4;
 __global__ __launch_bounds__(LIN_TRAIL_THREADS) void k_lin_trailing(Inst d, int k0, int b) {
-    __shared__ double u[16];
-    if (d.scal[4] != 0.0) return;
+    constexpr int CB = LIN_TRAIL_COLS, PER = 1024 / LIN_TRAIL_THREADS;
+    __shared__ double u[16][CB];
+    __shared__ double l11[16][17];
+    const double singular = d.scal[4];
     const int N = d.N, t = threadIdx.x;
     const int nr = N - k0;
-    const int j = k0 + b + blockIdx.x;
-    if (j > N) return;
-    double* cj = d.lin + (long)j * N + k0;  // rows from k0
+    const int j0 = k0 + b + blockIdx.x * CB;
+    const int nc = N + 1 - j0 < CB ? N + 1 - j0 : CB;
+    double* cj = d.lin + (long)j0 * N + k0;      // rows from k0, columns from j0
+    const double* lp = d.lin + (long)k0 * N + k0;  // the panel's factors
     const int* src = lin_perm(d);
-    constexpr int PER = 1024 / LIN_TRAIL_THREADS;
-    double v[PER];
+    double v[PER][CB];
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-        int q = t + m * LIN_TRAIL_THREADS;
-        v[m] = (q < nr && src[q] != q) ? cj[src[q]] : 0.0;
+        const int q = t + m * LIN_TRAIL_THREADS;
+        const int sq = q < nr ? src[q] : 0;
+        const int s = singular == 0.0 ? sq : 0;  // after a singular pivot the order may not be written
+#pragma unroll
+        for (int c = 0; c < CB; ++c) v[m][c] = q < nr && c < nc ? cj[(long)c * N + s] : 0.0;
+    }
+    double l[PER][16];  // every factor in flight at once
+#pragma unroll
+    for (int m = 0; m < PER; ++m) {
+        const int q = t + m * LIN_TRAIL_THREADS;
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) l[m][kk] = q >= 16 && q < nr ? lp[(long)kk * N + q] : 0.0;
+    }
+    l11[t & 15][t >> 4] = (t & 15) < b && (t >> 4) < b ? lp[(long)(t >> 4) * N + (t & 15)] : 0.0;  // [row][pivot]
+    if (singular != 0.0) return;
+    __syncthreads();  // every entry is read before one is written
+    if (t < WAVE) {
+        for (int m = 0; m < b - 1; ++m) {
+            const double f = l11[t & 15][m];
+            const bool below = t > m && t < b;
+#pragma unroll
+            for (int c = 0; c < CB; ++c) {
+                const double um = readlane_f64(v[0][c], m);
+                if (below) v[0][c] = v[0][c] - f * um;
+            }
+        }
+        if (t < b) {
+#pragma unroll
+            for (int c = 0; c < CB; ++c) u[t][c] = v[0][c];
+        }
     }
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-        int q = t + m * LIN_TRAIL_THREADS;
-        if (q < nr && src[q] != q) cj[q] = v[m];
-    }
-    __syncthreads();
-    if (t == 0) {
-        double uu[16];
-        for (int kk = 0; kk < b; ++kk) uu[kk] = cj[kk];
-        for (int kk = 1; kk < b; ++kk) {
-            double a = uu[kk];
-            for (int m = 0; m < kk; ++m) a = a - d.lin[(long)(k0 + m) * N + k0 + kk] * uu[m];
-            uu[kk] = a;
+        const int q = t + m * LIN_TRAIL_THREADS;
+        if (q >= 16 && q < nr) {  // rows below the panel: the panel has all its 16 columns
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk) {
+#pragma unroll
+                for (int c = 0; c < CB; ++c) v[m][c] = v[m][c] - l[m][kk] * u[kk][c];
+            }
         }
-        for (int kk = 0; kk < b; ++kk) {
-            u[kk] = uu[kk];
-            cj[kk] = uu[kk];
-        }
-    }
-    __syncthreads();
-    for (int q = b + t; q < nr; q += LIN_TRAIL_THREADS) {
-        double a = cj[q];
-        for (int kk = 0; kk < b; ++kk) a = a - d.lin[(long)(k0 + kk) * N + k0 + q] * u[kk];
-        cj[q] = a;
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+            if (q < nr && c < nc) cj[(long)c * N + q] = v[m][c];
     }
 }
 
-// Back substitution and the rest of the solve after the blocked factorization.
-// Shared memory: G [N] (+8), R [N], two product rows of linr_even(N + 64) (+16).
+// The back substitution after the blocked factorization: x (zero after a singular
+// pivot).  Shared memory: x [N] (+8), then the rows.
+template <int M>
+__global__ __launch_bounds__(BSUB_THREADS) void k_lin_back(Inst d, double* out) {
+    extern __shared__ double sh[];
+    const int N = d.N;
+    const bool solved = d.scal[4] == 0.0;
+    if (solved) back_substitute_group<M>(d.lin, N, sh, sh + linr_even(N + 8));
+    __syncthreads();
+    for (int i = threadIdx.x; i < N; i += BSUB_THREADS) out[i] = solved ? sh[i] : 0.0;
+}
+
+// Induced velocities of the N control points by the circulations in lin_solution
+// (induced_at's sums), into lin_induced.  A workgroup takes 64 of the 3 N (point,
+// component) chains: its waves bring the products of IND_ROWS columns into shared
+// memory, every load of a thread in flight at once, and one wave adds them in column
+// order, a chain per lane.  One workgroup for all chains waited on its own loads:
+// 1,020 strips, two calls and the strips' work around them: 538 -> 60 us.
+constexpr int IND_ROWS = 256;     // columns per turn: 128 KB of products
+constexpr int IND_THREADS = 1024;
+__global__ __launch_bounds__(IND_THREADS) void k_lin_induced(Inst d) {
+    extern __shared__ double prod[];  // [IND_ROWS][64]
+    constexpr int PER = IND_ROWS * WAVE / IND_THREADS;
+    const int N = d.N, t = threadIdx.x, lane = t & (WAVE - 1), w = t >> 6;
+    const int chain = blockIdx.x * WAVE + lane;  // 3 i + component
+    const int cc = chain < 3 * N ? chain : 3 * N - 1;
+    const double* G = lin_solution(d);
+    double sum = 0.0;
+    for (int j0 = 0; j0 < N; j0 += IND_ROWS) {
+        double f[PER], g[PER];
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const int j = min(j0 + w + u * (IND_THREADS / WAVE), N - 1);
+            f[u] = d.F[3L * N * j + cc];
+            g[u] = G[j];
+        }
+        __syncthreads();  // the previous turn's products are added
+#pragma unroll
+        for (int u = 0; u < PER; ++u) prod[(w + u * (IND_THREADS / WAVE)) * WAVE + lane] = f[u] * g[u];
+        __syncthreads();
+        if (w == 0) {
+            const int cnt = N - j0 < IND_ROWS ? N - j0 : IND_ROWS;
+            int q = 0;
+            for (; q + 16 <= cnt; q += 16) {
+                double v[16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) v[u] = prod[(q + u) * WAVE + lane];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) sum += v[u];
+            }
+            for (; q < cnt; ++q) sum += prod[q * WAVE + lane];
+        }
+    }
+    if (w == 0 && chain < 3 * N) {
+        double ind = d.fixed[chain];
+        ind += sum;
+        lin_induced(d)[chain] = ind;
+    }
+}
+
+// The strips' part between the two induced velocities: the corrected circulation, and
+// the first induced velocity kept for the strips that don't take the second.
+__global__ void k_lin_gamma(Inst d, int as_start) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= d.N) return;
+    const Strip s = load_strip(d, i);
+    const double g = lin_viscous_gamma(s, lin_solution(d)[i], lin_velocity(d, s, load3(lin_induced(d) + 3 * i), as_start));
+    lin_solution(d)[i] = g;
+}
+
+// The rest of the solve.  Shared memory: R [N].
 __global__ __launch_bounds__(1024) void k_lin_finish(Inst d, int as_start) {
     extern __shared__ double sh[];
-    const int N = d.N, t = threadIdx.x;
-    double* G = sh;
-    double* R = G + linr_even(N + 8);
-    double* pb = R + linr_even(N);
-    if (d.scal[4] != 0.0) {
-        if (t == 0)
-            for (int q = 0; q < N; ++q) G[q] = 0.0;
-    } else if (t < WAVE) {
-        back_substitute_wave_cm(d.lin, N, G, pb, (int)linr_even(N + 64));
-    }
-    __syncthreads();
-    const Strip s = load_strip(d, t < N ? t : N - 1);
-    lin_finish(d, s, G, R, as_start);
+    const int ic = (int)threadIdx.x < d.N ? threadIdx.x : d.N - 1;
+    const Strip s = load_strip(d, ic);
+    lin_outputs(d, s, lin_solution(d)[ic], lin_velocity(d, s, load3(lin_induced(d) + 3 * ic), as_start), sh, as_start);
 }
 
-// The blocked solve on a given system (checks of the elimination itself): the
-// back substitution of the factored d.lin into x; status = the singular step + 1
-// or 0.  Shared memory as k_lin_finish.
-__global__ __launch_bounds__(1024) void k_gauss_blocked_finish(Inst d, double* x, int* status) {
-    extern __shared__ double sh[];
-    const int N = d.N, t = threadIdx.x;
-    double* G = sh;
-    double* pb = G + linr_even(N + 8) + linr_even(N);
-    const int s = (int)d.scal[4];
-    if (s == 0 && t < WAVE) back_substitute_wave_cm(d.lin, N, G, pb, (int)linr_even(N + 64));
-    __syncthreads();
-    if (t == 0) *status = s;
-    for (int i = t; i < N; i += 1024) x[i] = s ? 0.0 : G[i];
-}
+// status = the singular step + 1 of the factored d.lin, or 0 (checks of the elimination itself).
+__global__ void k_gauss_status(Inst d, int* status) { *status = (int)d.scal[4]; }
 
 // ---------------------------------------------------------------------------
 // Forces (force_calculations.rs:322-548, forces_and_moments.rs:163-245,
@@ -3307,12 +3437,28 @@ static hipError_t launch_lin_blocked_factor(const Inst& d, hipStream_t st) {
     const int b = linearized_panel_width(N);
     for (int k0 = 0; k0 < N; k0 += b) {
         const int bb = N - k0 < b ? N - k0 : b;
-        const size_t shm = sizeof(double) * (size_t)(2 * LINP_W * LINP_SLOT + 2 * LINP_SLOT);
-        hipLaunchKernelGGL(k_lin_panel, dim3(1), dim3(LINP_T), shm, st, d, k0, bb);
+        const int rows = N - k0;
+        if (rows > LINP_T) hipLaunchKernelGGL(k_lin_panel<2>, dim3(1), dim3(LINP_T), 0, st, d, k0, bb);
+        else hipLaunchKernelGGL(k_lin_panel<1>, dim3(1), dim3((unsigned)((rows + WAVE - 1) / WAVE * WAVE)), 0, st, d, k0, bb);
         const unsigned cols = (unsigned)(N + 1 - k0 - bb);
-        hipLaunchKernelGGL(k_lin_trailing, dim3(cols), dim3(LIN_TRAIL_THREADS), 0, st, d, k0, bb);
+        hipLaunchKernelGGL(k_lin_trailing, dim3((cols + LIN_TRAIL_COLS - 1) / LIN_TRAIL_COLS), dim3(LIN_TRAIL_THREADS), 0, st, d, k0, bb);
     }
     return hipGetLastError();
+}
+
+template <int M>
+static hipError_t launch_lin_back_m(const Inst& d, double* x, hipStream_t st) {
+    const size_t shm = sizeof(double) * (size_t)(linr_even(d.N + 8) + bsub_doubles<M>());
+    hipError_t e = allow_shared((const void*)k_lin_back<M>, shm);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_lin_back<M>, dim3(1), dim3(BSUB_THREADS), shm, st, d, x);
+    return hipGetLastError();
+}
+// Columns per lane: as few as hold a row in one wave (the rows' fixed cost is the same).
+static hipError_t launch_lin_back(const Inst& d, double* x, hipStream_t st) {
+    if (d.N <= 4 * WAVE) return launch_lin_back_m<4>(d, x, st);
+    if (d.N <= 8 * WAVE) return launch_lin_back_m<8>(d, x, st);
+    return launch_lin_back_m<16>(d, x, st);
 }
 
 hipError_t launch_linearized(const Inst& d, int as_start, hipStream_t st) {
@@ -3333,10 +3479,18 @@ hipError_t launch_linearized(const Inst& d, int as_start, hipStream_t st) {
     hipLaunchKernelGGL(k_lin_assemble, dim3(blocks_for((long)N * (N + 1), 256)), dim3(256), 0, st, d);
     hipError_t eb = launch_lin_blocked_factor(d, st);
     if (eb != hipSuccess) return eb;
-    const size_t fin = sizeof(double) * (size_t)(linr_even(N + 8) + linr_even(N) + 2 * linr_even(N + 64) + 16);
-    hipError_t ef = allow_shared((const void*)k_lin_finish, fin);
-    if (ef != hipSuccess) return ef;
-    hipLaunchKernelGGL(k_lin_finish, dim3(1), dim3(1024), fin, st, d, as_start);
+    eb = launch_lin_back(d, lin_solution(d), st);
+    if (eb != hipSuccess) return eb;
+    const size_t prod = sizeof(double) * IND_ROWS * WAVE;
+    hipError_t ei = allow_shared((const void*)k_lin_induced, prod);
+    if (ei != hipSuccess) return ei;
+    const dim3 chains(blocks_for(3L * N, WAVE));
+    hipLaunchKernelGGL(k_lin_induced, chains, dim3(IND_THREADS), prod, st, d);
+    if (lin_viscous(d, as_start)) {
+        hipLaunchKernelGGL(k_lin_gamma, dim3(blocks_for(N, 64)), dim3(64), 0, st, d, as_start);
+        if (lin_second_velocity(d, as_start)) hipLaunchKernelGGL(k_lin_induced, chains, dim3(IND_THREADS), prod, st, d);
+    }
+    hipLaunchKernelGGL(k_lin_finish, dim3(1), dim3(1024), sizeof(double) * (size_t)N, st, d, as_start);
     return hipGetLastError();
 }
 
@@ -3359,10 +3513,9 @@ hipError_t launch_gauss_blocked(double* lin, double* scal, int N, double* x, int
     d.scal = scal;
     hipError_t e = launch_lin_blocked_factor(d, st);
     if (e != hipSuccess) return e;
-    const size_t fin = sizeof(double) * (size_t)(linr_even(N + 8) + linr_even(N) + 2 * linr_even(N + 64) + 16);
-    e = allow_shared((const void*)k_gauss_blocked_finish, fin);
+    e = launch_lin_back(d, x, st);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_gauss_blocked_finish, dim3(1), dim3(1024), fin, st, d, x, status);
+    hipLaunchKernelGGL(k_gauss_status, dim3(1), dim3(1), 0, st, d, status);
     return hipGetLastError();
 }
 

@@ -90,6 +90,19 @@ def test_random_systems(oracle, variant):
             check(oracle, A0, b, variant, "zero diagonal")
 
 
+@pytest.mark.parametrize("n", [255, 256, 257, 511, 512, 513, 530])
+def test_blocked_row_counts(oracle, n):
+    """The blocked form where its row layouts change: columns per lane of the back substitution (256,
+    512), rows per thread of the panel (512), with exchanges at every step and with many equal
+    magnitudes over all waves."""
+    rng = np.random.default_rng(9000 + n)
+    b = rng.standard_normal(n)
+    A = rng.standard_normal((n, n))
+    np.fill_diagonal(A, 0.0)
+    check(oracle, A, b, "blocked", "zero diagonal")
+    check(oracle, rng.integers(-2, 3, size=(n, n)).astype(np.float64), b, "blocked", "ties")
+
+
 @pytest.mark.parametrize("variant", [2, 4, "blocked"])
 def test_pivot_ties(oracle, variant):
     """Small integer entries: many equal magnitudes in the pivot column, so the

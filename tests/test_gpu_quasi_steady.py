@@ -81,6 +81,18 @@ def test_linearized_settings(oracle, solver):
     run_pair(oracle, js, [6.0, 2.0, 0], steps=2)
 
 
+@pytest.mark.parametrize("solver", [
+    {"Linearized": {"disable_viscous_corrections": True}},
+    {"Linearized": {"induced_velocity_correction_method": "NoCorrection"}},
+    {"Linearized": {"velocity_corrections": {"MaxInducedVelocityMagnitudeRatio": 0.05}}},
+    {"start_with_linearized_solution": True},
+])
+def test_linearized_settings_in_global_memory(oracle, solver):
+    """156 strips: the induced velocities and the strips' work in kernels of their own."""
+    js = S.wing_sails_quasi_steady(nr_strips=52, solver=solver)
+    run_pair(oracle, js, [6.0, 2.0, 0], steps=2)
+
+
 def test_quasi_steady_simple_iterative_and_linearized_start(oracle):
     base = {"max_iterations_per_time_step": 3000, "residual_tolerance_absolute": 1e-9,
             "strength_difference_tolerance": 1e-10}
