@@ -329,8 +329,8 @@ double sb_batch_last_step_ms(const sb_batch* b);
 int sb_batch_reset(sb_batch* b);
 
 /* Kernel variants of the batched pair sums (no counterpart in the reference):
- * fixed_per = panels per compute wave per block of the fixed-velocity kernel
- * (1, 2, 3), targets_tile = panel records per LDS tile of the self-induction
+ * fixed_per = fours of panels per compute wave per block of the fixed-velocity
+ * kernel (1, 2, 3), targets_tile = panel records per LDS tile of the self-induction
  * kernel (64, 128, 256).  Results do not depend on them (every target keeps its
  * ascending panel order). */
 int sb_batch_set_tuning(sb_batch* b, int fixed_per, int targets_tile);

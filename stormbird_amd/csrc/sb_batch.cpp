@@ -201,7 +201,7 @@ struct sb_batch {
         cap_fixed_jobs = 0;
         cap_target_jobs = 0;
         for (auto& s : sims) {
-            cap_fixed_jobs += (s->N + 63) / 64;
+            cap_fixed_jobs += (s->N + FIXED_JOB_TARGETS - 1) / FIXED_JOB_TARGETS;
             long np = (long)s->P * (s->M + 1);
             long end = std::min<long>(s->setup.wake.end_index, np);
             cap_target_jobs += (end + 255) / 256;
@@ -349,7 +349,7 @@ struct sb_batch {
         for (int i = 0; i < n; ++i) {
             const Inst& d = h_inst[2 * n + i];
             long len = (long)d.N * std::max(d.nz_rows - 1, 0);
-            for (int tb = 0; tb < (d.N + 63) / 64; ++tb) fj.push_back({len, int2{i, tb}});
+            for (int tb = 0; tb < (d.N + FIXED_JOB_TARGETS - 1) / FIXED_JOB_TARGETS; ++tb) fj.push_back({len, int2{i, tb}});
         }
         std::stable_sort(fj.begin(), fj.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
         for (size_t k = 0; k < fj.size(); ++k) h_jobs[k] = fj[k].second;
@@ -364,7 +364,7 @@ struct sb_batch {
         bd.n_fixed_jobs = (int)fj.size();
         bd.n_target_jobs = (int)nt;
         fixed_work = 0.0;
-        for (const auto& f : fj) fixed_work += 64.0 * (double)f.first;
+        for (const auto& f : fj) fixed_work += (double)FIXED_JOB_TARGETS * (double)f.first;
         target_work = 0.0;
         for (long k = 0; k < nt; ++k) {
             const Inst& d = h_inst[3 * n + h_jobs[cap_fixed_jobs + k].x];
@@ -536,7 +536,7 @@ struct sb_batch {
 
     // Times every variant of the batched pair kernels on the batch's own last-step state
     // (outputs saved and restored, so the state is unchanged) and applies the fastest.
-    // timings: kb_fixed for 1, 2, 3 panels per wave, then kb_targets for 64, 128, 256
+    // timings: kb_fixed for 1, 2, 3 fours of panels per wave, then kb_targets for 64, 128, 256
     // records per tile (ms, -1 where a kernel had no work).
     void autotune(double* timings, int reps, long max_jobs) {
         if (quasi) throw std::invalid_argument("the autotuner covers dynamic batches");

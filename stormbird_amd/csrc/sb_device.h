@@ -129,6 +129,9 @@ struct McBuffers {
     int tmap_span = 0;  // span points per wave of the map (0: flat order)
 };
 
+// Control points per job of the batched fixed velocities (kb_fixed).
+constexpr int FIXED_JOB_TARGETS = 16;
+
 // Scratch of the two-pass few-target sum (k_terms + k_fold_terms): one chunk
 // of per-pair terms [3][n_targets][row] and the running sums [3][n_targets].
 struct FoldBuffers {
@@ -223,7 +226,7 @@ struct BatchDev {
     int n_target_jobs = 0;
     unsigned* counters = nullptr;       // device [2] job-queue heads, zero between launches
     int fixed_grid = 0, target_grid = 0;  // persistent workgroups
-    int fixed_per = 3;            // kb_fixed: panels per compute wave per block (1, 2, 3)
+    int fixed_per = 1;            // kb_fixed: fours of panels per compute wave per block (1, 2, 3)
     int targets_tile = 256;       // kb_targets: panel records per LDS tile (64, 128, 256)
     int stage_near = 0;           // kb_targets: 1 when every self-induced instance has ring-edge
                                   // geometry (near-field data staged with the records)

@@ -2917,29 +2917,32 @@ __device__ inline int next_job(unsigned* head, int* slot) {
 }
 
 // Fixed velocities of many instances (frozen_wake.rs:189-261).  Job = one
-// instance's 64 control points (lane = target) over its panels of rows >= 1,
-// run by one 16-wave workgroup (a whole CU).  Fifteen compute waves evaluate
-// the panels of a 45-panel block (three consecutive panels each) into one
-// half of a double-buffered LDS term array while the last wave adds the
-// previous block's terms, component by component, in ascending panel order:
-// one barrier per block, and every target sees the same sequence of additions
-// as the one-target fold (a skipped panel adds +0, which leaves a sum that
-// started at +0 unchanged).  Panel records are read with scalar loads (the
-// address is wave-uniform), the next block's across the barrier, so the
-// compute waves use no LDS for them.  Jobs are taken longest first from a
-// queue by persistent workgroups.
-constexpr int COOP_WAVES = 16;
-constexpr int FX_COMPUTE = 15;  // compute waves; wave 15 folds
+// instance's FX_TARGETS control points over its panels of rows >= 1, run by one
+// workgroup.  The compute waves' lanes are 16 targets x 4 consecutive panels; they
+// evaluate a block of panels (4 PER consecutive ones each) into one half of a
+// double-buffered LDS term array while the last wave adds the previous block's terms,
+// a lane per (component, target) chain, in ascending panel order: one barrier per
+// block, and every target sees the same sequence of additions as the one-target fold
+// (a skipped panel, and one past the end, adds +0, which leaves a sum that started at
+// +0 unchanged).  The next block's records are loaded across the barrier.  Jobs are
+// taken longest first from a queue by persistent workgroups.
+// 16 targets per job, not the 64 of a wave: a job is one instance's whole wake in
+// order, so the longest instance's jobs bound the launch, and fewer lanes are padding
+// (96 polar instances, the largest 372 strips x 1,000 rows: step 18.8 -> 9.6 ms; 400
+// instances of up to 600 rows, where the queue evens out either way: 22.1 -> 20.9).
+constexpr int FX_WAVES = 16;  // a job on a whole CU (8: 10.4 and 20.3 ms on those batches, 4: 18.9 and 21.1)
+constexpr int FX_COMPUTE = FX_WAVES - 1;  // compute waves; the last wave folds
+constexpr int FX_TARGETS = FIXED_JOB_TARGETS;
+constexpr int FX_SUB = WAVE / FX_TARGETS; // panels side by side in a wave
 
-// PER panels per compute wave per block (1, 2 or 3; the autotuner picks it):
-// blocks of 15 PER panels, a double-buffered term array of 2 x 15 PER x 1.5 KiB.
+// PER x 4 panels per compute wave per block (PER 1, 2 or 3; the autotuner picks it).
 template <int MODE, int SYM, int PER>
-__global__ __launch_bounds__(1024) void kb_fixed(const Inst* I, const int2* __restrict__ jobs, int n_jobs,
-                                                 unsigned* head) {
-    constexpr int FX_BLOCK = FX_COMPUTE * PER;
-    constexpr int FOLD_CHUNK = FX_BLOCK / 5;  // the fold's loads run one chunk ahead of its adds
-    static_assert(FX_BLOCK % FOLD_CHUNK == 0, "the fold reads full blocks in chunks");
-    __shared__ double T[2][FX_BLOCK][3][WAVE];  // 46,080 B per panel per wave
+__global__ __launch_bounds__(FX_WAVES* WAVE) __attribute__((amdgpu_waves_per_eu(4))) void kb_fixed(
+    const Inst* I, const int2* __restrict__ jobs, int n_jobs, unsigned* head) {
+    constexpr int ROWS = FX_COMPUTE * PER;
+    constexpr int FX_BLOCK = ROWS * FX_SUB;  // panels per block
+    constexpr int CS = WAVE + 8;             // the components' chains in different banks
+    __shared__ double T[2][ROWS][3][CS];
     __shared__ int slot;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
     const int lane = threadIdx.x % WAVE;
@@ -2948,44 +2951,40 @@ __global__ __launch_bounds__(1024) void kb_fixed(const Inst* I, const int2* __re
         if (j >= n_jobs) break;
         int2 jb = jobs[j];
         const Inst d = I[jb.x];
-        int t = jb.y * WAVE + lane;
+        int t = jb.y * FX_TARGETS + lane % FX_TARGETS;
         int tc = t < d.N ? t : d.N - 1;
-        V3 x = load3(d.geo + d.gl.ctrl + 3 * tc);
-        int wt = d.neglect_self ? d.wing_of[tc] : -1;
-        const long p_begin = d.N, p_end = (long)d.N * d.nz_rows;
-        const long nblk = p_end > p_begin ? (p_end - p_begin + FX_BLOCK - 1) / FX_BLOCK : 0;
-        double acc = 0.0;
+        const int pb = d.N, pe = d.N * d.nz_rows;
+        const int nblk = pe > pb ? (pe - pb + FX_BLOCK - 1) / FX_BLOCK : 0;
         if (wave < FX_COMPUTE) {
-            ScalarRecs recs = (ScalarRecs)d.rec;
-            const int pb = (int)p_begin, pe = (int)p_end;
-            const int mine = pb + wave * PER;  // first panel of this wave in block 0
+            const V3 x = load3(d.geo + d.gl.ctrl + 3 * tc);
+            const int wt = d.neglect_self ? d.wing_of[tc] : -1;
+            int k0 = pb + wave * PER * FX_SUB + lane / FX_TARGETS;  // the lane's first panel of the block
             PanelRec r[PER];
             if (nblk > 0) {
 #pragma unroll
-                for (int q = 0; q < PER; ++q) r[q] = scalar_rec(recs, mine + q < pe ? mine + q : pe - 1);
+                for (int q = 0; q < PER; ++q) r[q] = d.rec[min(k0 + q * FX_SUB, pe - 1)];
             }
-            for (int b = 0; b <= (int)nblk; ++b) {
-                if (b < (int)nblk) {
+            for (int b = 0; b <= nblk; ++b) {
+                if (b < nblk) {
                     const int buf = b & 1;
-                    const int k0 = mine + b * FX_BLOCK;
                     V3 term[PER];
                     if constexpr (SYM == 0 && MODE != MODE_FP32_KAHAN) {
-                        // far-field terms of the three panels, interleaved; then the
+                        // far-field terms of the panels, interleaved; then the
                         // lanes that need the general evaluation
                         bool ok[PER];
 #pragma unroll
                         for (int q = 0; q < PER; ++q) ok[q] = far_fast<MODE>(r[q], x, term[q]);
 #pragma unroll
                         for (int q = 0; q < PER; ++q)
-                            if (!ok[q]) term[q] = panel_unit<MODE>(d, r[q], k0 + q < pe ? k0 + q : pe - 1, x);
+                            if (!ok[q]) term[q] = panel_unit<MODE>(d, r[q], min(k0 + q * FX_SUB, pe - 1), x);
                     } else {
 #pragma unroll
                         for (int q = 0; q < PER; ++q)
-                            term[q] = pair_unit<MODE, SYM>(d, r[q], k0 + q < pe ? k0 + q : pe - 1, x);
+                            term[q] = pair_unit<MODE, SYM>(d, r[q], min(k0 + q * FX_SUB, pe - 1), x);
                     }
 #pragma unroll
                     for (int q = 0; q < PER; ++q) {
-                        const int k = k0 + q;
+                        const int k = k0 + q * FX_SUB;
                         bool skip = k >= pe || r[q].strength == 0.0 ||
                                     (d.neglect_self && d.wing_of[k % d.N] == wt);
                         V3 u = skip ? V3{0.0, 0.0, 0.0} : term[q] * r[q].strength;
@@ -2994,49 +2993,36 @@ __global__ __launch_bounds__(1024) void kb_fixed(const Inst* I, const int2* __re
                         T[buf][kl][1][lane] = u.y;
                         T[buf][kl][2][lane] = u.z;
                     }
-                    // records of the next block, loaded across the barrier
-                    const int kn = k0 + FX_BLOCK;
+                    k0 += FX_BLOCK;
 #pragma unroll
-                    for (int q = 0; q < PER; ++q) r[q] = scalar_rec(recs, kn + q < pe ? kn + q : pe - 1);
+                    for (int q = 0; q < PER; ++q) r[q] = d.rec[min(k0 + q * FX_SUB, pe - 1)];
                 }
                 __syncthreads();
             }
         } else {
-            double ay = 0.0, az = 0.0;
-            for (long b = 0; b <= nblk; ++b) {
+            const int c = lane / FX_TARGETS < 3 ? lane / FX_TARGETS : 2;
+            double acc = 0.0;
+            for (int b = 0; b <= nblk; ++b) {
                 if (b > 0) {
-                    const int buf = (int)((b - 1) & 1);
-                    const long base = p_begin + (b - 1) * FX_BLOCK;
-                    const int cnt = (int)(p_end - base < FX_BLOCK ? p_end - base : FX_BLOCK);
-                    if (cnt == FX_BLOCK) {
-                        // a full block: loads issued a chunk ahead of the adds
+                    const double* src = &T[(b - 1) & 1][0][c][lane % FX_TARGETS];
+                    constexpr int AHEAD = 3;  // rows of terms read before they are added
+                    static_assert(ROWS % AHEAD == 0, "whole groups of rows");
 #pragma unroll
-                        for (int q0 = 0; q0 < FX_BLOCK; q0 += FOLD_CHUNK) {
-                            double vx[FOLD_CHUNK], vy[FOLD_CHUNK], vz[FOLD_CHUNK];
+                    for (int q0 = 0; q0 < ROWS; q0 += AHEAD) {
+                        double v[AHEAD][FX_SUB];
 #pragma unroll
-                            for (int i = 0; i < FOLD_CHUNK; ++i) {
-                                vx[i] = T[buf][q0 + i][0][lane];
-                                vy[i] = T[buf][q0 + i][1][lane];
-                                vz[i] = T[buf][q0 + i][2][lane];
-                            }
+                        for (int i = 0; i < AHEAD; ++i)
 #pragma unroll
-                            for (int i = 0; i < FOLD_CHUNK; ++i) {
-                                acc = acc + vx[i];
-                                ay = ay + vy[i];
-                                az = az + vz[i];
-                            }
-                        }
-                    } else {
-                        for (int q = 0; q < cnt; ++q) {
-                            acc = acc + T[buf][q][0][lane];
-                            ay = ay + T[buf][q][1][lane];
-                            az = az + T[buf][q][2][lane];
-                        }
+                            for (int u = 0; u < FX_SUB; ++u) v[i][u] = src[(q0 + i) * 3 * CS + u * FX_TARGETS];
+#pragma unroll
+                        for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+                            for (int u = 0; u < FX_SUB; ++u) acc = acc + v[i][u];
                     }
                 }
                 __syncthreads();
             }
-            if (t < d.N) store3(d.fixed + 3 * t, V3{acc, ay, az});
+            if (lane < 3 * FX_TARGETS && t < d.N) d.fixed[3 * t + c] = acc;
         }
     }
 }
@@ -3748,8 +3734,8 @@ hipError_t launch_batch_panels(const BatchDev& b, int shift, hipStream_t st) {
 
 template <int MODE, int SYM, int PER>
 static void launch_kb_fixed(const BatchDev& b, hipStream_t st) {
-    hipLaunchKernelGGL((kb_fixed<MODE, SYM, PER>), dim3(b.fixed_grid), dim3(COOP_WAVES * WAVE), 0, st, b.inst,
-                       b.fixed_jobs, b.n_fixed_jobs, b.counters);
+    hipLaunchKernelGGL((kb_fixed<MODE, SYM, PER>), dim3(b.fixed_grid), dim3(FX_WAVES * WAVE), 0, st, b.inst, b.fixed_jobs,
+                       b.n_fixed_jobs, b.counters);
 }
 
 template <int MODE, int SYM>
@@ -3863,7 +3849,7 @@ static int resident_groups(K kernel, int threads) {
 
 template <int MODE, int SYM>
 static int fixed_groups(int per) {
-    const int th = COOP_WAVES * WAVE;
+    const int th = FX_WAVES * WAVE;
     if (per == 1) return resident_groups(kb_fixed<MODE, SYM, 1>, th);
     if (per == 2) return resident_groups(kb_fixed<MODE, SYM, 2>, th);
     return resident_groups(kb_fixed<MODE, SYM, 3>, th);

@@ -70,6 +70,34 @@ def test_batch_equals_alone_fast():
     run_pair(sb.MODE_FAST, 6)
 
 
+@pytest.mark.parametrize("neglect", [False, True])
+@pytest.mark.parametrize("symmetry", [None, "Z"])
+def test_fixed_velocity_jobs_at_their_edges(neglect, symmetry):
+    """Control points below, at and above a job's 16, wakes from 2 rows (fewer panels than a block of
+    the fixed-velocity kernel) up: the batch gives the bits of the instances alone, in every variant."""
+    import json
+
+    setups = []
+    for sails, strips, rows in [(1, 1, 2), (1, 15, 3), (1, 16, 9), (1, 17, 6), (3, 5, 12), (2, 17, 8), (4, 4, 2)]:
+        js, case = S.four_sail_free_wake(nr_panels=rows, nr_strips=strips, ratio=0.0)
+        d = json.loads(js)
+        d["line_force_model"]["wing_builders"] = d["line_force_model"]["wing_builders"][:sails]
+        wake = d["simulation_settings"]["Dynamic"]["wake"]
+        if neglect:
+            wake["neglect_self_induced_velocities"] = True
+        if symmetry:
+            wake["symmetry_condition"] = symmetry
+        setups.append(json.dumps(d))
+    batch, alone = sb.Batch(setups), [sb.Simulation(js) for js in setups]
+    parts = [S.uniform_freestream(a.nr_freestream_points(), case["velocity"]) for a in alone]
+    for k in range(13):
+        batch.set_tuning(1 + k % 3, 64)
+        rb = batch.do_step(times=0.2 * k, time_steps=0.2, freestream_velocity=np.concatenate(parts))
+        for i, a in enumerate(alone):
+            ra = a.do_step(time=0.2 * k, time_step=0.2, freestream_velocity=parts[i])
+            compare_results(rb[i], ra, exact=True, where=f"step {k} instance {i}")
+
+
 def test_batch_instance_matches_oracle(oracle):
     rng = np.random.default_rng(11)
     setups, cases = [], []
