@@ -226,7 +226,7 @@ struct BatchDev {
     int n_target_jobs = 0;
     unsigned* counters = nullptr;       // device [2] job-queue heads, zero between launches
     int fixed_grid = 0, target_grid = 0;  // persistent workgroups
-    int fixed_per = 1;            // kb_fixed: fours of panels per compute wave per block (1, 2, 3)
+    int fixed_per = 3;            // kb_fixed: fours of panels per compute wave per block (1, 2, 3)
     int targets_tile = 256;       // kb_targets: panel records per LDS tile (64, 128, 256)
     int stage_near = 0;           // kb_targets: 1 when every self-induced instance has ring-edge
                                   // geometry (near-field data staged with the records)

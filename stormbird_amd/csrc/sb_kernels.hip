@@ -15,6 +15,8 @@
 // a refined reciprocal square root instead.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "sb_device.h"
 #include "sb_wind.h"
 #include "sb_mlp.h"
@@ -2916,35 +2918,104 @@ __device__ inline int next_job(unsigned* head, int* slot) {
     return __builtin_amdgcn_readfirstlane(*slot);
 }
 
-// Fixed velocities of many instances (frozen_wake.rs:189-261).  Job = one
-// instance's FX_TARGETS control points over its panels of rows >= 1, run by one
-// workgroup.  The compute waves' lanes are 16 targets x 4 consecutive panels; they
+// ---- ordered pair sums, 16 targets per workgroup ----
+// The panels [pb, pe) onto the workgroup's FX_TARGETS targets, each target's terms added
+// in ascending panel order.  The compute waves' lanes are 16 targets x 4 consecutive
+// panels (x: the lane's target; wt: its wing, or -1 where its own wing counts); they
 // evaluate a block of panels (4 PER consecutive ones each) into one half of a
 // double-buffered LDS term array while the last wave adds the previous block's terms,
-// a lane per (component, target) chain, in ascending panel order: one barrier per
-// block, and every target sees the same sequence of additions as the one-target fold
-// (a skipped panel, and one past the end, adds +0, which leaves a sum that started at
-// +0 unchanged).  The next block's records are loaded across the barrier.  Jobs are
-// taken longest first from a queue by persistent workgroups.
-// 16 targets per job, not the 64 of a wave: a job is one instance's whole wake in
-// order, so the longest instance's jobs bound the launch, and fewer lanes are padding
-// (96 polar instances, the largest 372 strips x 1,000 rows: step 18.8 -> 9.6 ms; 400
-// instances of up to 600 rows, where the queue evens out either way: 22.1 -> 20.9).
-constexpr int FX_WAVES = 16;  // a job on a whole CU (8: 10.4 and 20.3 ms on those batches, 4: 18.9 and 21.1)
+// a lane per (component, target) chain: one barrier per block, and every target sees
+// the same sequence of additions as the one-target fold (a skipped panel, and one past
+// the end, adds +0, which leaves a sum that started at +0 unchanged).  The next block's
+// records are loaded across the barrier.  Returns chain lane % 16 of component lane / 16
+// in lanes 0-47 of the last wave.  Every thread of the workgroup calls it with the
+// same panels.
+// A sum over panels is a chain, so the parallel work is in the targets: 16 of them on a
+// whole CU serve where 64 or 256 per workgroup leave the chip with too few waves, or
+// with a few that run long.
+constexpr int FX_WAVES = 16;              // a job on a whole CU (8: 10.4 ms on the polar batch below, 4: 18.9)
 constexpr int FX_COMPUTE = FX_WAVES - 1;  // compute waves; the last wave folds
 constexpr int FX_TARGETS = FIXED_JOB_TARGETS;
 constexpr int FX_SUB = WAVE / FX_TARGETS; // panels side by side in a wave
+constexpr int FX_STRIDE = WAVE + 8;       // the components' chains in different banks
+template <int PER>
+struct FxTerms {
+    double t[2][FX_COMPUTE * PER][3][FX_STRIDE];
+};
+template <int MODE, int SYM, int PER>
+__device__ inline double ordered_block_sum(const Inst& d, V3 x, int wt, int pb, int pe, FxTerms<PER>& T) {
+    constexpr int ROWS = FX_COMPUTE * PER;
+    constexpr int FX_BLOCK = ROWS * FX_SUB;  // panels per block
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int lane = threadIdx.x % WAVE;
+    const int nblk = pe > pb ? (pe - pb + FX_BLOCK - 1) / FX_BLOCK : 0;
+    double acc = 0.0;
+    if (wave < FX_COMPUTE) {
+        int k = pb + wave * PER * FX_SUB + lane / FX_TARGETS;  // the lane's panel
+        PanelRec next{};
+        if (nblk > 0) next = d.rec[min(k, pe - 1)];
+        for (int b = 0; b <= nblk; ++b) {
+            if (b < nblk) {
+                double(*row)[3][FX_STRIDE] = T.t[b & 1] + wave * PER;
+#pragma nounroll
+                for (int q = 0; q < PER; ++q) {
+                    const PanelRec r = next;
+                    V3 term;
+                    if constexpr (SYM == 0 && MODE != MODE_FP32_KAHAN) {
+                        // the far-field term; then the lanes that need the general evaluation
+                        if (!far_fast<MODE>(r, x, term)) term = panel_unit<MODE>(d, r, min(k, pe - 1), x);
+                    } else {
+                        term = pair_unit<MODE, SYM>(d, r, min(k, pe - 1), x);
+                    }
+                    const bool skip = k >= pe || r.strength == 0.0 || (wt >= 0 && d.wing_of[k % d.N] == wt);
+                    const V3 u = skip ? V3{0.0, 0.0, 0.0} : term * r.strength;
+                    k += q + 1 < PER ? FX_SUB : FX_BLOCK - (PER - 1) * FX_SUB;
+                    next = d.rec[min(k, pe - 1)];
+                    row[q][0][lane] = u.x;
+                    row[q][1][lane] = u.y;
+                    row[q][2][lane] = u.z;
+                }
+            }
+            __syncthreads();
+        }
+    } else {
+        const int c = lane / FX_TARGETS < 3 ? lane / FX_TARGETS : 2;
+        for (int b = 0; b <= nblk; ++b) {
+            if (b > 0) {
+                const double* src = &T.t[(b - 1) & 1][0][c][lane % FX_TARGETS];
+                constexpr int AHEAD = 3;  // rows of terms read before they are added
+                static_assert(ROWS % AHEAD == 0, "whole groups of rows");
+#pragma unroll
+                for (int q0 = 0; q0 < ROWS; q0 += AHEAD) {
+                    double v[AHEAD][FX_SUB];
+#pragma unroll
+                    for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+                        for (int u = 0; u < FX_SUB; ++u) v[i][u] = src[(q0 + i) * 3 * FX_STRIDE + u * FX_TARGETS];
+#pragma unroll
+                    for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+                        for (int u = 0; u < FX_SUB; ++u) acc = acc + v[i][u];
+                }
+            }
+            __syncthreads();
+        }
+    }
+    return acc;
+}
 
+// Fixed velocities of many instances (frozen_wake.rs:189-261).  Job = one
+// instance's FX_TARGETS control points over its panels of rows >= 1.  Jobs are
+// taken longest first from a queue by persistent workgroups (96 polar instances, the
+// largest 372 strips x 1,000 rows: step 18.8 -> 9.6 ms against jobs of 64 control
+// points with a wave-uniform panel; 400 instances of up to 600 rows, where the queue
+// evens out either way: 22.1 -> 20.9).
 // PER x 4 panels per compute wave per block (PER 1, 2 or 3; the autotuner picks it).
 template <int MODE, int SYM, int PER>
 __global__ __launch_bounds__(FX_WAVES* WAVE) __attribute__((amdgpu_waves_per_eu(4))) void kb_fixed(
     const Inst* I, const int2* __restrict__ jobs, int n_jobs, unsigned* head) {
-    constexpr int ROWS = FX_COMPUTE * PER;
-    constexpr int FX_BLOCK = ROWS * FX_SUB;  // panels per block
-    constexpr int CS = WAVE + 8;             // the components' chains in different banks
-    __shared__ double T[2][ROWS][3][CS];
+    __shared__ FxTerms<PER> T;
     __shared__ int slot;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
     const int lane = threadIdx.x % WAVE;
     for (;;) {
         int j = next_job(head, &slot);
@@ -2953,77 +3024,31 @@ __global__ __launch_bounds__(FX_WAVES* WAVE) __attribute__((amdgpu_waves_per_eu(
         const Inst d = I[jb.x];
         int t = jb.y * FX_TARGETS + lane % FX_TARGETS;
         int tc = t < d.N ? t : d.N - 1;
-        const int pb = d.N, pe = d.N * d.nz_rows;
-        const int nblk = pe > pb ? (pe - pb + FX_BLOCK - 1) / FX_BLOCK : 0;
-        if (wave < FX_COMPUTE) {
-            const V3 x = load3(d.geo + d.gl.ctrl + 3 * tc);
-            const int wt = d.neglect_self ? d.wing_of[tc] : -1;
-            int k0 = pb + wave * PER * FX_SUB + lane / FX_TARGETS;  // the lane's first panel of the block
-            PanelRec r[PER];
-            if (nblk > 0) {
-#pragma unroll
-                for (int q = 0; q < PER; ++q) r[q] = d.rec[min(k0 + q * FX_SUB, pe - 1)];
-            }
-            for (int b = 0; b <= nblk; ++b) {
-                if (b < nblk) {
-                    const int buf = b & 1;
-                    V3 term[PER];
-                    if constexpr (SYM == 0 && MODE != MODE_FP32_KAHAN) {
-                        // far-field terms of the panels, interleaved; then the
-                        // lanes that need the general evaluation
-                        bool ok[PER];
-#pragma unroll
-                        for (int q = 0; q < PER; ++q) ok[q] = far_fast<MODE>(r[q], x, term[q]);
-#pragma unroll
-                        for (int q = 0; q < PER; ++q)
-                            if (!ok[q]) term[q] = panel_unit<MODE>(d, r[q], min(k0 + q * FX_SUB, pe - 1), x);
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < PER; ++q)
-                            term[q] = pair_unit<MODE, SYM>(d, r[q], min(k0 + q * FX_SUB, pe - 1), x);
-                    }
-#pragma unroll
-                    for (int q = 0; q < PER; ++q) {
-                        const int k = k0 + q * FX_SUB;
-                        bool skip = k >= pe || r[q].strength == 0.0 ||
-                                    (d.neglect_self && d.wing_of[k % d.N] == wt);
-                        V3 u = skip ? V3{0.0, 0.0, 0.0} : term[q] * r[q].strength;
-                        const int kl = wave * PER + q;
-                        T[buf][kl][0][lane] = u.x;
-                        T[buf][kl][1][lane] = u.y;
-                        T[buf][kl][2][lane] = u.z;
-                    }
-                    k0 += FX_BLOCK;
-#pragma unroll
-                    for (int q = 0; q < PER; ++q) r[q] = d.rec[min(k0 + q * FX_SUB, pe - 1)];
-                }
-                __syncthreads();
-            }
-        } else {
-            const int c = lane / FX_TARGETS < 3 ? lane / FX_TARGETS : 2;
-            double acc = 0.0;
-            for (int b = 0; b <= nblk; ++b) {
-                if (b > 0) {
-                    const double* src = &T[(b - 1) & 1][0][c][lane % FX_TARGETS];
-                    constexpr int AHEAD = 3;  // rows of terms read before they are added
-                    static_assert(ROWS % AHEAD == 0, "whole groups of rows");
-#pragma unroll
-                    for (int q0 = 0; q0 < ROWS; q0 += AHEAD) {
-                        double v[AHEAD][FX_SUB];
-#pragma unroll
-                        for (int i = 0; i < AHEAD; ++i)
-#pragma unroll
-                            for (int u = 0; u < FX_SUB; ++u) v[i][u] = src[(q0 + i) * 3 * CS + u * FX_TARGETS];
-#pragma unroll
-                        for (int i = 0; i < AHEAD; ++i)
-#pragma unroll
-                            for (int u = 0; u < FX_SUB; ++u) acc = acc + v[i][u];
-                    }
-                }
-                __syncthreads();
-            }
-            if (lane < 3 * FX_TARGETS && t < d.N) d.fixed[3 * t + c] = acc;
-        }
+        const V3 x = load3(d.geo + d.gl.ctrl + 3 * tc);
+        const double acc = ordered_block_sum<MODE, SYM, PER>(d, x, d.neglect_self ? d.wing_of[tc] : -1, d.N,
+                                                             d.N * d.nz_rows, T);
+        if (threadIdx.x >= FX_COMPUTE * WAVE && lane < 3 * FX_TARGETS && t < d.N)
+            d.fixed[3 * t + lane / FX_TARGETS] = acc;
+    }
+}
+
+// Self-induction of one instance with too few wake points to fill the GPU 256 to a
+// workgroup: 16 per workgroup.  Three fours of panels per wave per block: a wave with
+// near-field lanes takes five times as long, and longer blocks even that out (3 sails x
+// 27 strips x 533 rows EXACT 11.8 ms per step, with one four 12.3; 25.5 with 256 points
+// per workgroup).
+constexpr int FEW_PER = 3;
+template <int MODE, int SYM>
+__global__ __launch_bounds__(FX_WAVES* WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_targets_few(
+    Inst d, const double* __restrict__ targets, long n_targets, long n_panels, double* __restrict__ out, int add) {
+    __shared__ FxTerms<FEW_PER> T;
+    const int lane = threadIdx.x % WAVE;
+    const long t = (long)blockIdx.x * FX_TARGETS + lane % FX_TARGETS;
+    const V3 x = load3(targets + 3 * (t < n_targets ? t : n_targets - 1));
+    const double acc = ordered_block_sum<MODE, SYM, FEW_PER>(d, x, -1, 0, (int)n_panels, T);
+    if (threadIdx.x >= FX_COMPUTE * WAVE && lane < 3 * FX_TARGETS && t < n_targets) {
+        double* o = out + 3 * t + lane / FX_TARGETS;
+        *o = add ? *o + acc : acc;
     }
 }
 
@@ -3059,6 +3084,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
 }
 
+// The same jobs for batches with too few wake points to fill the GPU 256 to a workgroup:
+// a workgroup takes a sixteenth of a job.
+template <int MODE, int SYM>
+__global__ __launch_bounds__(FX_WAVES* WAVE) __attribute__((amdgpu_waves_per_eu(4))) void kb_targets_few(
+    const Inst* I, const int2* __restrict__ jobs, int n_jobs, unsigned* head) {
+    constexpr int PARTS = 256 / FX_TARGETS;
+    __shared__ FxTerms<FEW_PER> T;
+    __shared__ int slot;
+    const int lane = threadIdx.x % WAVE;
+    for (;;) {
+        const int j = next_job(head, &slot);
+        if (j >= n_jobs * PARTS) break;
+        const int2 jb = jobs[j / PARTS];
+        const Inst d = I[jb.x];
+        const long np = (long)d.P * (d.M + 1);
+        const long end = d.end_index < np ? d.end_index : np;
+        const long t0 = (long)jb.y * 256 + (j % PARTS) * FX_TARGETS, t = t0 + lane % FX_TARGETS;
+        if (t0 >= end) continue;
+        const V3 x = load3(d.pts + 3 * (t < end ? t : end - 1));
+        const double acc = ordered_block_sum<MODE, SYM, FEW_PER>(d, x, -1, 0, d.N * d.nz_rows, T);
+        if (threadIdx.x >= FX_COMPUTE * WAVE && lane < 3 * FX_TARGETS && t < end)
+            d.vel[3 * t + lane / FX_TARGETS] += acc;
+    }
+}
 
 // ---- learned warm start: per-strip features and the initial guess ----
 // Features of strip i (wing strips [a, b)): for o = -4..4, strip j = i + o
@@ -3552,6 +3601,18 @@ hipError_t launch_velocity_copy(const Inst& d, hipStream_t st) {
     return hipGetLastError();
 }
 
+static long cu_count() {
+    static std::atomic<long> cached{0};
+    long c = cached.load(std::memory_order_relaxed);
+    if (c == 0) {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+            c = v;
+        cached.store(c, std::memory_order_relaxed);
+    }
+    return c;
+}
+
 template <int MODE, int SYM, bool NB>
 static int mc_slots_for() {
     int per_cu = 0, cus = 0, dev = 0;
@@ -3591,6 +3652,16 @@ static hipError_t launch_targets_t(const Inst& d, const double* targets, long n_
             hipLaunchKernelGGL((k_targets_mc<MODE, SYM, false>), dim3((unsigned)grid), dim3(256), 0, st, d, targets,
                                n_targets, out, add, pl);
     } else {
+        if constexpr (MODE != MODE_FP32_KAHAN) {
+            // up to 1.5 workgroups of 256 per CU (there the two take the same time within 7 %
+            // either way, measured at 450 of them: EXACT 87.6 ms against 91.8, FAST 71.1
+            // against 66.2; at 176: 11.8 against 25.5 and 9.7 against 18.9)
+            if (!tmap && 2 * n_jobs <= 3 * cu_count()) {
+                hipLaunchKernelGGL((k_targets_few<MODE, SYM>), dim3(blocks_for(n_targets, FX_TARGETS)),
+                                   dim3(FX_WAVES * WAVE), 0, st, d, targets, n_targets, n_panels, out, add);
+                return hipGetLastError();
+            }
+        }
         if (nb)
             hipLaunchKernelGGL((k_targets<MODE, SYM, true>), dim3((unsigned)n_jobs), dim3(256), 0, st, d, targets,
                                n_targets, n_panels, out, add, tmap);
@@ -3819,6 +3890,14 @@ static void launch_kb_targets(const BatchDev& b, hipStream_t st) {
 
 template <int MODE, int SYM>
 static void launch_kb_targets_tile(const BatchDev& b, hipStream_t st) {
+    // few: up to 3 workgroups of 256 per CU in EXACT (12 ships, 936 of them: 50.6 ms per
+    // step against 50.0; 8 ships, 624: 34.2 against 42.7; 4: 17.9 against 30.0), up to 1.5
+    // in FAST, whose sweep gains more from the wave-uniform panel
+    if (2 * b.n_target_jobs <= (MODE == MODE_EXACT ? 6 : 3) * cu_count()) {
+        hipLaunchKernelGGL((kb_targets_few<MODE, SYM>), dim3((unsigned)cu_count()), dim3(FX_WAVES * WAVE), 0, st, b.inst,
+                           b.target_jobs, b.n_target_jobs, b.counters + 1);
+        return;
+    }
     if (b.targets_tile == 64) launch_kb_targets<MODE, SYM, 64>(b, st);
     else if (b.targets_tile == 128) launch_kb_targets<MODE, SYM, 128>(b, st);
     else launch_kb_targets<MODE, SYM, 256>(b, st);

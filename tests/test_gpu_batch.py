@@ -98,6 +98,43 @@ def test_fixed_velocity_jobs_at_their_edges(neglect, symmetry):
             compare_results(rb[i], ra, exact=True, where=f"step {k} instance {i}")
 
 
+@pytest.mark.parametrize("mode", [sb.MODE_EXACT, sb.MODE_FAST])
+def test_self_induction_kernels_on_both_sides_of_their_rules(mode):
+    """16 wake points per workgroup or 256 (single instances: at most 384 workgroups of 256 on 256 CUs;
+    batches: 768 in EXACT): the same wake step through every route gives the same bits.  A target map
+    keeps a single instance on the 256-point kernel."""
+    rows = 590  # 4 x 41 x 591 points: 379 workgroups of 256
+    js, case = S.four_sail_free_wake(nr_panels=rows)
+    alone = sb.Simulation(js, mode=mode)
+    tiled = sb.Simulation(js, mode=mode)
+    tiled.target_tiling = 8
+    batches = [sb.Batch([js] * n, mode=mode) for n in (1, 2, 3)]  # 379, 758, 1,137 workgroups
+    data = np.load(S.DEVELOPED_FOUR_SAIL)
+    p = data["points"].reshape(2001, -1, 3)[:rows + 1].astype(np.float64).reshape(-1, 3)
+    g = data["strengths"].reshape(2000, -1)[:rows].astype(np.float64)
+    u = np.tile(np.asarray(case["velocity"]), (p.shape[0], 1))
+    fs = S.uniform_freestream(alone.nr_freestream_points(), case["velocity"])
+
+    def load(sim):
+        sim.set_wake_state(p, u, g.ravel(), rows)
+        sim.previous_circulation_strength = g[0]
+
+    for sim in (alone, tiled):
+        load(sim)
+        sim.do_step(time=1.0, time_step=0.2, freestream_velocity=fs)
+    want = alone.get_wake_state()
+    got = [tiled.get_wake_state()]
+    for b in batches:
+        b.do_step(times=0.0, time_steps=0.2, freestream_velocity=np.concatenate([fs] * len(b.instances)))
+        for sim in b.instances:
+            load(sim)
+        b.do_step(times=1.0, time_steps=0.2, freestream_velocity=np.concatenate([fs] * len(b.instances)))
+        got += [sim.get_wake_state() for sim in b.instances]
+    for i, w in enumerate(got):
+        for key in ("points", "velocities", "strengths"):
+            assert same(w[key], want[key]), f"route {i}: wake {key}"
+
+
 def test_batch_instance_matches_oracle(oracle):
     rng = np.random.default_rng(11)
     setups, cases = [], []
