@@ -1870,71 +1870,63 @@ __device__ inline void lin_finish(const Inst& d, const Strip& s, double* G, doub
 }
 
 // ---- one-workgroup form (small N) -------------------------------------------
-// T threads in 8 column groups x T/8 row groups: thread (rg, cg) holds rows
-// r = rg + s T/8 (s < R) and columns j = cg + 8 c (c < C = 4 CB; the right-hand
-// side is column N) of the augmented matrix in registers for the whole
-// elimination, so a pivot-row value read from shared memory serves R rows.  Row
-// exchanges are not carried out: every wave keeps the logical position of every
-// row (lanes hold rows l, l + 64, ...) and which rows have been pivots.  Per pivot k:
-//   - column k of every row is read from shared memory (cst, published at step k - 1);
-//   - every wave reduces it on its own: the largest magnitude among the rows not
-//     yet used, NaN excluded, ties to the lower logical position; the row at
-//     position k when that row holds NaN (linalg.rs:58-64 scans positions
-//     k + 1.. with a strict >, so a NaN at position k is never replaced);
-//   - the pivot row's threads publish its columns >= k (prow, [8][C + 2]), and
-//     each thread forms its factors f = a[r][k] / pivot; barrier;
-//   - every row subtracts f * prow[j] entry by entry in the blocks of 4 register
-//     columns that hold a column >= k (the rows already used as pivots and the
-//     entries left of column k + 1 take harmless updates: they are never read
-//     again), wave 0 copies the pivot row into U (row-major, logical position k),
-//     and the owners of column k + 1 publish it; barrier.
-// Wave 0 then back-substitutes.
+// The augmented matrix in shared memory, column-major with an odd leading dimension
+// (rows and columns both read without bank conflicts), eliminated in panels of LINR_B
+// columns:
+//   - wave 0 factors the panel in its registers, lane l holding rows l + 64 s below the
+//     panel's top.  Rows are not exchanged meanwhile: every row keeps its logical
+//     position.  A pivot is a search over the wave (the largest magnitude, NaN excluded,
+//     ties to the lower position; the row at the pivot's position when that holds NaN:
+//     linalg.rs:58-64 scans the positions behind it with a strict >), the pivot row by
+//     readlane, a division and the panel's own updates: no barrier and no trip through
+//     shared memory.  The rows are written back at their positions, with their sources;
+//   - barrier; every wave takes columns behind the panel (the right-hand side is column
+//     N): its rows gathered from their sources, then a - f * p for the panel's pivots in
+//     order, p handed on by readlane (row m of the panel is final after m updates);
+//   - barrier.
+// Wave 0 then back-substitutes.  The pivots' chain bounds it (a pivot costs ~1,200
+// cycles; with every wave searching, the pivot row published through shared memory and
+// two barriers per pivot it was 3,300): 120 strips, kernel 271 -> 219 us (elimination 165
+// -> 107, back substitution 62); 1,024 instances of 8-128 strips 815 -> 600.
+constexpr int LINR_B = 8;
 template <int V>
-struct LinrV;  // <threads, rows per thread, blocks of 4 columns per thread, 64-row slices of the pivot search>
+struct LinrV;  // <threads, 64-row slices>
 template <>
 struct LinrV<1> {
-    static constexpr int T = 256, R = 2, CB = 3, MS = 1;  // N <= 64
+    static constexpr int T = 256, RL = 1;  // N <= 64
 };
 template <>
 struct LinrV<2> {
-    static constexpr int T = 256, R = 4, CB = 4, MS = 2;  // N <= 127
+    static constexpr int T = 512, RL = 2;  // N <= 128
 };
 template <>
 struct LinrV<3> {
-    static constexpr int T = 256, R = 4, CB = 5, MS = 2;  // N <= 128
-};
-template <>
-struct LinrV<4> {
-    static constexpr int T = 512, R = 3, CB = 5, MS = 3;  // N <= 159 (160 KB of shared memory: N <= 139)
+    static constexpr int T = 512, RL = 3;  // N <= 192 (160 KB of shared memory: N <= 139)
 };
 template <int V>
-SB_HD inline bool linr_fits(int N) {
-    using P = LinrV<V>;
-    return N >= 1 && N <= P::T / 8 * P::R && N + 1 <= 32 * P::CB && N <= 64 * P::MS;
-}
-// Shared memory (doubles): U [N][N + 1] (+8), G [N] (+8), R [N], cst (column k of
-// every row, [N + 1] with a spare slot; later the back substitution's two product
-// rows), prow [8][C + 2].  Every region starts on a 16-byte boundary.
+SB_HD inline bool linr_fits(int N) { return N >= 1 && N <= WAVE * LinrV<V>::RL; }
+// Shared memory (doubles): matrix [N + 1][ld], G [N] (+8), R [N], the back
+// substitution's two product rows, the rows' sources [N] (ints), the singular step.
+// Every region starts on a 16-byte boundary.
 struct LinrLayout {
-    long G, R, cst, prow, total;
+    long G, R, prod, src, total;
+    int ld;
     int pstride;  // product row stride of the back substitution
 };
 SB_HD inline long linr_even(long v) { return (v + 1) & ~1L; }
 constexpr int LINR_PS = 3;  // product slots per lane of the back substitution (N <= 192)
-template <int V>
 SB_HD inline LinrLayout linr_layout(int N) {
     LinrLayout L;
+    L.ld = N | 1;
     L.pstride = (int)(N + 40 > 64 * LINR_PS ? linr_even(N + 40) : 64 * LINR_PS);
-    L.G = (long)N * (N + 1) + 8;
+    L.G = linr_even((long)(N + 1) * L.ld);
     L.R = L.G + linr_even(N + 8);
-    L.cst = L.R + linr_even(N);
-    const long cst = N + 1 > 2L * L.pstride + 16 ? N + 1 : 2L * L.pstride + 16;
-    L.prow = L.cst + linr_even(cst);
-    L.total = L.prow + 8L * (4 * LinrV<V>::CB + 2);
+    L.prod = L.R + linr_even(N);
+    L.src = L.prod + 2L * L.pstride + 16;
+    L.total = L.src + linr_even((N + 1) / 2 + 1);
     return L;
 }
-template <int V>
-SB_HD inline long linr_shared_doubles(int N) { return linr_layout<V>(N).total; }
+SB_HD inline long linr_shared_doubles(int N) { return linr_layout(N).total; }
 
 template <int CTRL>
 __device__ inline double dpp_f64(double v) {
@@ -1960,8 +1952,32 @@ __device__ inline int wave_min_i32(int v) {
                min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
-// linalg.rs:92-101 by one wave over the row-major upper triangle U (logical
-// rows, leading dimension N + 1), N <= 64 PS.  Every lane runs the same ordered
+// The lane of the largest v >= 0 (NaN and negative values never win), ties to the
+// smallest key; -1 when no lane has one.  The high words are reduced first: one
+// 32-bit instruction per level, and they alone usually name the lane.
+__device__ inline int wave_argmax(double v, int key) {
+    const bool in = v >= 0.0;
+    const unsigned h = in ? (unsigned)__double2hiint(v) + 1u : 0u;
+    unsigned m = h;
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 1>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 2>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 4>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 8>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_BCAST15, 0xa>(0, (int)m));
+    m = max(m, (unsigned)dpp_i32<DPP_BCAST31, 0xc>(0, (int)m));
+    m = (unsigned)__builtin_amdgcn_readlane((int)m, WAVE - 1);
+    if (m == 0u) return -1;
+    unsigned long long top = __ballot(h == m);
+    if (top & (top - 1)) {
+        const bool cand = h == m;
+        const double best = wave_max_f64(cand ? v : -1.0);
+        const int k = wave_min_i32(cand && v == best ? key : 0x7fffffff);
+        top = __ballot(cand && v == best && key == k);
+    }
+    return (int)__builtin_ctzll(top);
+}
+// linalg.rs:92-101 by one wave over the factored matrix U (column-major, leading
+// dimension ld, column N the right-hand side), N <= 64 PS.  Every lane runs the same ordered
 // sum sum = ((0 + u[i][i+1] x[i+1]) + u[i][i+2] x[i+2]) + ..., reading the
 // products u[i][j] x[j], j >= i + 2, from shared memory (pb, two rows of pstride
 // >= max(N + 40, 64 PS)) in groups of 16: lane t forms the products of row i - 1
@@ -1970,22 +1986,21 @@ __device__ inline int wave_min_i32(int v) {
 // it starts at +0.0 and cannot become -0.0.  (Fewer instructions per row, not
 // fewer latencies, is what shortens this loop: one wave issues all of it.)
 template <int PS>
-__device__ inline void back_substitute_wave(const double* U, int N, double* x, double* pb, int pstride) {
+__device__ inline void back_substitute_wave(const double* U, int ld, int N, double* x, double* pb, int pstride) {
     const int lane = threadIdx.x & (WAVE - 1);
-    const long ld = N + 1;
-    double xprev = (U[(N - 1) * ld + N] - 0.0) / U[(N - 1) * ld + N - 1];
+    double xprev = (U[N * ld + N - 1] - 0.0) / U[(N - 1) * ld + N - 1];
     x[N - 1] = xprev;
     for (int i = N - 2; i >= 0; --i) {
-        const double* row = U + i * ld;
-        const double di = row[i], bi = row[N], u1 = row[i + 1];
+        const double* row = U + i;
+        const double di = row[i * ld], bi = row[N * ld], u1 = row[(i + 1) * ld];
         const int lenp = i >= 1 ? N - i - 1 : 0;  // products of row i - 1
-        const double* rowp = row - (i >= 1 ? ld : 0);
+        const double* rowp = row - (i >= 1 ? 1 : 0);
         double pr[PS];
 #pragma unroll
         for (int s = 0; s < PS; ++s) {
             const int t = lane + WAVE * s;
             const int j = min(i + 1 + t, N - 1);
-            const double p = rowp[j] * x[j];
+            const double p = rowp[j * ld] * x[j];
             pr[s] = t < lenp ? p : 0.0;
         }
         double sum = 0.0 + u1 * xprev;
@@ -2043,206 +2058,188 @@ struct DenseSrc {  // a row-major N x N matrix and its right-hand side
     __device__ double entry(Row, int r, int j) const { return j < N ? A[(long)r * N + j] : b[r]; }
 };
 
+// Columns [k0, k0 + b) factored by one wave; returns 0 or the singular step + 1.
+// Pivot KK as a template, so that every register index is fixed.
+template <int RL>
+struct LinrPanel {
+    double a[RL][LINR_B];
+    int pos[RL];    // logical position of each row below the panel's top
+    bool done[RL];  // a pivot already, or past the matrix
+};
+template <int KK, int RL>
+__device__ __forceinline__ int linr_panel_steps(int k0, int b, LinrPanel<RL>& st) {
+    if constexpr (KK < LINR_B) {
+        if (KK >= b) return 0;
+        double v = -1.0;
+        int key = 0x7fffffff, slot = 0;
+        bool nan = false;  // the row at the pivot's position holds NaN
+#pragma unroll
+        for (int s = 0; s < RL; ++s) {
+            const double vs = fabs(st.a[s][KK]);
+            const bool take = !st.done[s] && (vs > v || (vs == v && st.pos[s] < key));  // NaN never is
+            v = take ? vs : v;
+            key = take ? st.pos[s] : key;
+            slot = take ? s : slot;
+            nan = nan | (!st.done[s] && st.pos[s] == KK && vs != vs);
+        }
+        int win = wave_argmax(v, key);
+        const unsigned long long stuck = __ballot(nan);
+        if (stuck) {
+            win = (int)__builtin_ctzll(stuck);
+            key = KK;
+#pragma unroll
+            for (int s = 0; s < RL; ++s)
+                if (!st.done[s] && st.pos[s] == KK) slot = s;
+        }
+        double p[LINR_B];
+#pragma unroll
+        for (int c = KK; c < LINR_B; ++c) {
+            double e = st.a[0][c];
+#pragma unroll
+            for (int s = 1; s < RL; ++s) e = slot == s ? st.a[s][c] : e;
+            p[c] = readlane_f64(e, win);
+        }
+        const int ppos = __builtin_amdgcn_readlane(key, win);
+        if (fabs(p[KK]) < 1e-12) return k0 + KK + 1;
+        const bool mine = (int)(threadIdx.x & (WAVE - 1)) == win;
+#pragma unroll
+        for (int s = 0; s < RL; ++s) {
+            const bool pivot = mine && slot == s;
+            const bool moved = !pivot && !st.done[s] && st.pos[s] == KK;
+            st.pos[s] = pivot ? KK : moved ? ppos : st.pos[s];
+            st.done[s] = st.done[s] | pivot;
+            const double f = st.a[s][KK] / p[KK];
+            if (!st.done[s]) {
+#pragma unroll
+                for (int c = KK + 1; c < LINR_B; ++c) st.a[s][c] = st.a[s][c] - f * p[c];
+                st.a[s][KK] = f;
+            }
+        }
+        return linr_panel_steps<KK + 1, RL>(k0, b, st);
+    }
+    return 0;
+}
+
+// The panel at `top` (row k0 of column k0) by one wave: factors and pivot rows written back
+// at their positions, the rows' sources to src.
+template <int RL>
+__device__ inline int linr_panel(double* top, int ld, int k0, int nr, int b, int* src) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    LinrPanel<RL> st;
+#pragma unroll
+    for (int s = 0; s < RL; ++s) {
+        const int q = lane + WAVE * s;
+        st.pos[s] = q;
+        st.done[s] = q >= nr;
+#pragma unroll
+        for (int c = 0; c < LINR_B; ++c) st.a[s][c] = q < nr && c < b ? top[c * ld + q] : 0.0;
+    }
+    const int singular = linr_panel_steps<0, RL>(k0, b, st);
+    if (singular) return singular;
+#pragma unroll
+    for (int s = 0; s < RL; ++s) {
+        const int q = lane + WAVE * s;
+        if (q < nr) {
+#pragma unroll
+            for (int c = 0; c < LINR_B; ++c)
+                if (c < b) top[c * ld + st.pos[s]] = st.a[s][c];
+            src[st.pos[s]] = q;
+        }
+    }
+    return 0;
+}
+
+// The columns behind the panel: exchanges and updates, a wave per column (NW waves).
+template <int RL, int NW>
+__device__ inline void linr_trailing(double* A, const double* top, int ld, int N, int k0, int nr, int b, const int* src) {
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
+    double l[RL][LINR_B];
+    int from[RL];
+#pragma unroll
+    for (int s = 0; s < RL; ++s) {
+        const int q = lane + WAVE * s;
+        from[s] = q < nr ? src[q] : 0;
+#pragma unroll
+        for (int m = 0; m < LINR_B; ++m) l[s][m] = q < nr && m < b ? top[m * ld + q] : 0.0;
+    }
+    constexpr int CC = 2;  // columns of a wave side by side
+    for (int j0 = k0 + b + w; j0 <= N; j0 += CC * NW) {
+        double v[CC][RL];
+#pragma unroll
+        for (int c = 0; c < CC; ++c)
+#pragma unroll
+            for (int s = 0; s < RL; ++s) v[c][s] = A[min(j0 + c * NW, N) * ld + k0 + from[s]];
+#pragma unroll
+        for (int m = 0; m < LINR_B; ++m) {
+            if (m < b) {
+#pragma unroll
+                for (int c = 0; c < CC; ++c) {
+                    const double um = readlane_f64(v[c][0], m);
+                    const double below = v[c][0] - l[0][m] * um;
+                    v[c][0] = lane > m ? below : v[c][0];
+#pragma unroll
+                    for (int s = 1; s < RL; ++s) v[c][s] = v[c][s] - l[s][m] * um;
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < CC; ++c)
+#pragma unroll
+            for (int s = 0; s < RL; ++s)
+                if (lane + WAVE * s < nr && j0 + c * NW <= N) A[(j0 + c * NW) * ld + k0 + lane + WAVE * s] = v[c][s];
+    }
+}
+
 // Solves the system on one workgroup of LinrV<V>::T threads; the solution goes to
 // G of the layout.  Returns 0, or k + 1 when the pivot of step k is below 1e-12 in
 // magnitude (linalg.rs:67-71; G is then not written).  Ends with a barrier.
 template <int V, class Src>
-__device__ inline int gauss_regs(int N, const Src& src, double* sh) {
+__device__ inline int gauss_lds(int N, const Src& system, double* sh) {
     using P = LinrV<V>;
-    constexpr int T = P::T, R = P::R, CB = P::CB, MS = P::MS;
-    constexpr int CG = 8, RG = T / CG, C = 4 * CB;
-    constexpr int US = (8 * C + WAVE - 1) / WAVE;  // wave 0's slots for the columns <= N
-    const LinrLayout L = linr_layout<V>(N);
-    const int t = threadIdx.x, lane = t & (WAVE - 1);
-    const int rg = t >> 3, cg = t & 7;
-    double* U = sh;
-    double* G = sh + L.G;
-    double* cst = sh + L.cst;
-    double* prow = sh + L.prow;
-    double* prq = prow + cg * (C + 2);
-    const long ld = N + 1;
-    const int nbu = (N + 1 + 31) >> 5;  // blocks of 4 register columns that hold a column <= N
-    int rs[R];                          // this thread's rows; N (a spare slot of cst) past the end
-#pragma unroll
-    for (int s = 0; s < R; ++s) rs[s] = rg + RG * s < N ? rg + RG * s : N;
-    double a[R][C];
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        const int r = rg + RG * s;
-        const bool own = r < N;
-        const auto qr = src.row(own ? r : N - 1);
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int j = cg + CG * c;
-            a[s][c] = own && j <= N ? src.entry(qr, r, j) : 0.0;
-        }
+    constexpr int T = P::T, RL = P::RL, NW = T / WAVE;
+    constexpr int RW = RL == 3 ? 256 : WAVE * RL;  // rows per turn of the assembly
+    const LinrLayout L = linr_layout(N);
+    const int t = threadIdx.x, lane = t & (WAVE - 1), w = t >> 6, ld = L.ld;
+    double* A = sh;
+    int* src = (int*)(sh + L.src);
+    int* sing = src + N;
+    if (t % RW < N) {
+        const int r = t % RW;
+        const auto q = system.row(r);
+        for (int j = t / RW; j <= N; j += T / RW) A[j * ld + r] = system.entry(q, r, j);
     }
-    if (cg == 0) {
-#pragma unroll
-        for (int s = 0; s < R; ++s) cst[rs[s]] = a[s][0];
-    }
-    int wpos[MS];
-    bool wdone[MS];
-#pragma unroll
-    for (int sl = 0; sl < MS; ++sl) {
-        wpos[sl] = lane + WAVE * sl;
-        wdone[sl] = false;
-    }
-    int singular = 0;
+    if (t == 0) *sing = 0;
     __syncthreads();
-    for (int k = 0; k < N; ++k) {
-        double v[MS];
-#pragma unroll
-        for (int sl = 0; sl < MS; ++sl) {
-            const int row = lane + WAVE * sl;
-            v[sl] = cst[row < N ? row : N - 1];
-        }
-        double fa[R];
-#pragma unroll
-        for (int s = 0; s < R; ++s) fa[s] = cst[rs[s]];
-        double mm = -1.0;
-#pragma unroll
-        for (int sl = 0; sl < MS; ++sl) {
-            const bool cand = lane + WAVE * sl < N && !wdone[sl];
-            mm = fmax(mm, cand ? fabs(v[sl]) : -1.0);
-        }
-        const double M = wave_max_f64(mm);
-        int key = 0x7fffffff;  // logical position * 1024 + row
-        int rk = -1;           // row at logical position k
-        bool nank = false;
-#pragma unroll
-        for (int sl = 0; sl < MS; ++sl) {
-            const int row = lane + WAVE * sl;
-            const bool cand = row < N && !wdone[sl];
-            const int kk = wpos[sl] * 1024 + row;
-            if (cand && fabs(v[sl]) == M && kk < key) key = kk;
-            if (cand && wpos[sl] == k) {
-                rk = row;
-                nank = v[sl] != v[sl];
-            }
-        }
-        const int K = wave_min_i32(key);
-        {
-            const unsigned long long hit = __ballot(rk >= 0);
-            const int src_lane = (int)__builtin_ctzll(hit);
-            rk = __builtin_amdgcn_readlane(rk, src_lane);
-            nank = __builtin_amdgcn_readlane((int)nank, src_lane) != 0;
-        }
-        int pr = K & 1023, ppos = K >> 10;
-        if (nank) {
-            pr = rk;
-            ppos = k;
-        }
-        pr = __builtin_amdgcn_readfirstlane(pr);
-        const int ps = pr >> 6;
-        double vsel = v[0];
-#pragma unroll
-        for (int sl = 1; sl < MS; ++sl)
-            if (ps == sl) vsel = v[sl];
-        const double piv = readlane_f64(vsel, pr & (WAVE - 1));
-        // a singular pivot is recorded and the remaining steps run on (their results
-        // are not used): the loop keeps one uniform exit
-        if (fabs(piv) < 1e-12 && !singular) singular = k + 1;
-#pragma unroll
-        for (int sl = 0; sl < MS; ++sl) {
-            const int row = lane + WAVE * sl;
-            if (row == pr) {
-                wpos[sl] = k;
-                wdone[sl] = true;
-            } else if (row == rk) {
-                wpos[sl] = ppos;
-            }
-        }
-        const int b0 = k >> 5;  // blocks that hold a column >= k
-        if (rg == pr % RG) {    // the pivot row's threads
-            const int sp = pr / RG;
-#pragma unroll
-            for (int s = 0; s < R; ++s) {
-                if (s == sp) {
-#pragma unroll
-                    for (int b = 0; b < CB; ++b) {
-                        if (b >= b0 && b < nbu) {
-                            double2* o = (double2*)(prq + 4 * b);
-                            o[0] = make_double2(a[s][4 * b], a[s][4 * b + 1]);
-                            o[1] = make_double2(a[s][4 * b + 2], a[s][4 * b + 3]);
-                        }
-                    }
-                }
-            }
-        }
-        // the factors, formed after the pivot row's stores are issued and before the barrier
-        double f[R];
-#pragma unroll
-        for (int s = 0; s < R; ++s) {
-            f[s] = fa[s] / piv;
-            asm volatile("" ::"v"(f[s]));
+    for (int k0 = 0; k0 < N; k0 += LINR_B) {
+        const int nr = N - k0, b = nr < LINR_B ? nr : LINR_B;
+        double* top = A + k0 * ld + k0;  // row k0 of column k0
+        const bool one = RL > 1 && nr <= WAVE;  // the rows left fit one slice
+        if (w == 0) {
+            const int singular = one ? linr_panel<1>(top, ld, k0, nr, b, src) : linr_panel<RL>(top, ld, k0, nr, b, src);
+            if (singular && lane == 0) *sing = singular;
         }
         __syncthreads();
-        double2 w[C / 2];
-#pragma unroll
-        for (int b = 0; b < CB; ++b) {
-            if (b < nbu) {
-                const double2* s2 = (const double2*)(prq + 4 * b);
-                w[2 * b] = s2[0];
-                w[2 * b + 1] = s2[1];
-            }
-        }
-        double uc[US];
-        if (t < WAVE) {  // wave 0 copies the pivot row into U (logical row k)
-#pragma unroll
-            for (int sl = 0; sl < US; ++sl) {
-                const int j = lane + WAVE * sl;
-                uc[sl] = j <= N ? prow[(j & 7) * (C + 2) + (j >> 3)] : 0.0;
-            }
-        }
-#pragma unroll
-        for (int b = 0; b < CB; ++b) {
-            if (b >= b0 && b < nbu) {
-#pragma unroll
-                for (int s = 0; s < R; ++s) {
-                    a[s][4 * b] = a[s][4 * b] - f[s] * w[2 * b].x;
-                    a[s][4 * b + 1] = a[s][4 * b + 1] - f[s] * w[2 * b].y;
-                    a[s][4 * b + 2] = a[s][4 * b + 2] - f[s] * w[2 * b + 1].x;
-                    a[s][4 * b + 3] = a[s][4 * b + 3] - f[s] * w[2 * b + 1].y;
-                }
-            }
-        }
-        if (k + 1 < N && cg == ((k + 1) & 7)) {  // publish column k + 1
-            const int c1 = (k + 1) >> 3;
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                if (c == c1) {
-#pragma unroll
-                    for (int s = 0; s < R; ++s) cst[rs[s]] = a[s][c];
-                }
-            }
-        }
-        if (t < WAVE) {
-#pragma unroll
-            for (int sl = 0; sl < US; ++sl) {
-                const int j = lane + WAVE * sl;
-                if (j <= N) U[k * ld + j] = uc[sl];
-            }
-        }
+        if (*sing) return *sing;  // uniform; written before the barrier only
+        if (one) linr_trailing<1, NW>(A, top, ld, N, k0, nr, b, src);
+        else linr_trailing<RL, NW>(A, top, ld, N, k0, nr, b, src);
         __syncthreads();
     }
-    if (singular) return singular;
-    if (t < WAVE) {
-        if (N <= 128) back_substitute_wave<2>(U, N, G, cst, L.pstride);
-        else back_substitute_wave<LINR_PS>(U, N, G, cst, L.pstride);
+    if (w == 0) {
+        if (N <= 128) back_substitute_wave<2>(A, ld, N, sh + L.G, sh + L.prod, L.pstride);
+        else back_substitute_wave<LINR_PS>(A, ld, N, sh + L.G, sh + L.prod, L.pstride);
     }
     __syncthreads();
     return 0;
 }
 
 template <int V>
-__device__ inline void linearized_reg_body(const Inst& d, double* sh, int as_start) {
+__device__ inline void linearized_lds_body(const Inst& d, double* sh, int as_start) {
     const int N = d.N;
     const int t = threadIdx.x;
-    const LinrLayout L = linr_layout<V>(N);
+    const LinrLayout L = linr_layout(N);
     double* G = sh + L.G;
     double* R = sh + L.R;
-    const int singular = gauss_regs<V>(N, LinSystemSrc{&d}, sh);
+    const int singular = gauss_lds<V>(N, LinSystemSrc{&d}, sh);
     if (singular) {
         if (t == 0) {
             for (int qq = 0; qq < N; ++qq) G[qq] = 0.0;
@@ -2253,9 +2250,9 @@ __device__ inline void linearized_reg_body(const Inst& d, double* sh, int as_sta
     lin_finish(d, load_strip(d, t < N ? t : N - 1), G, R, as_start);
 }
 template <int V>
-__global__ __launch_bounds__(LinrV<V>::T) void k_linearized(Inst d, int as_start) {
+__global__ __launch_bounds__(LinrV<V>::T) __attribute__((amdgpu_waves_per_eu(V == 1 ? 4 : 2))) void k_linearized(Inst d, int as_start) {
     extern __shared__ double sh[];
-    linearized_reg_body<V>(d, sh, as_start);
+    linearized_lds_body<V>(d, sh, as_start);
 }
 
 // The one-workgroup solve on a given system (checks of the elimination itself):
@@ -2263,8 +2260,8 @@ __global__ __launch_bounds__(LinrV<V>::T) void k_linearized(Inst d, int as_start
 template <int V>
 __global__ __launch_bounds__(LinrV<V>::T) void k_gauss_dense(const double* A, const double* b, int N, double* x, int* status) {
     extern __shared__ double sh[];
-    const int s = gauss_regs<V>(N, DenseSrc{A, b, N}, sh);
-    const double* G = sh + linr_layout<V>(N).G;
+    const int s = gauss_lds<V>(N, DenseSrc{A, b, N}, sh);
+    const double* G = sh + linr_layout(N).G;
     if (threadIdx.x == 0) *status = s;
     for (int i = threadIdx.x; i < N; i += LinrV<V>::T) x[i] = s ? 0.0 : G[i];
 }
@@ -2331,30 +2328,6 @@ struct LinPanelState {
     int pos[R];    // logical position of each row in the panel
     bool done[R];  // a pivot already, or past the matrix
 };
-// The lane of the largest v >= 0 (NaN and negative values never win), ties to the
-// smallest key; -1 when no lane has one.  The high words are reduced first: one
-// 32-bit instruction per level, and they alone usually name the lane.
-__device__ inline int wave_argmax(double v, int key) {
-    const bool in = v >= 0.0;
-    const unsigned h = in ? (unsigned)__double2hiint(v) + 1u : 0u;
-    unsigned m = h;
-    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 1>(0, (int)m));
-    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 2>(0, (int)m));
-    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 4>(0, (int)m));
-    m = max(m, (unsigned)dpp_i32<DPP_ROW_SHR + 8>(0, (int)m));
-    m = max(m, (unsigned)dpp_i32<DPP_BCAST15, 0xa>(0, (int)m));
-    m = max(m, (unsigned)dpp_i32<DPP_BCAST31, 0xc>(0, (int)m));
-    m = (unsigned)__builtin_amdgcn_readlane((int)m, WAVE - 1);
-    if (m == 0u) return -1;
-    unsigned long long top = __ballot(h == m);
-    if (top & (top - 1)) {
-        const bool cand = h == m;
-        const double best = wave_max_f64(cand ? v : -1.0);
-        const int k = wave_min_i32(cand && v == best ? key : 0x7fffffff);
-        top = __ballot(cand && v == best && key == k);
-    }
-    return (int)__builtin_ctzll(top);
-}
 // Pivot KK of the panel (a template, so that every register index is fixed).
 // Returns false at a singular pivot (recorded in scal[4]).
 template <int KK, int R>
@@ -2871,11 +2844,13 @@ __global__ void kb_horseshoe_factors(const Inst* I, const long* off, int n) {
 }
 
 // One workgroup per instance (the one-workgroup Linearized form).
+// The instances with above < N <= upto.
 template <int V>
-__global__ __launch_bounds__(LinrV<V>::T) void kb_linearized(const Inst* I, int as_start) {
+__global__ __launch_bounds__(LinrV<V>::T) __attribute__((amdgpu_waves_per_eu(V == 1 ? 4 : 2))) void kb_linearized(const Inst* I, int above, int upto, int as_start) {
     extern __shared__ double sh[];
     const Inst d = I[blockIdx.x];
-    linearized_reg_body<V>(d, sh, as_start);
+    if (d.N <= above || d.N > upto) return;
+    linearized_lds_body<V>(d, sh, as_start);
 }
 
 // Singular-pivot flags of every instance (scal[4]) into flags[n], then cleared.
@@ -3411,28 +3386,23 @@ static hipError_t allow_shared(const void* fn, size_t bytes) {
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-// One-workgroup variants (LinrV): a variant applies when the rows and columns
-// fit its threads' registers and its shared memory fits the device.
+// One-workgroup variants (LinrV): a variant applies when the rows fit its wave's
+// registers and the matrix the device's shared memory.
 template <int V>
 static bool linr_ok(int N) {
-    return linr_fits<V>(N) && (long)sizeof(double) * linr_shared_doubles<V>(N) <= lds_limit_bytes();
+    return linr_fits<V>(N) && (long)sizeof(double) * linr_shared_doubles(N) <= lds_limit_bytes();
 }
 static bool linr_variant_ok(int v, int N) {
     switch (v) {
         case 1: return linr_ok<1>(N);
         case 2: return linr_ok<2>(N);
         case 3: return linr_ok<3>(N);
-        case 4: return linr_ok<4>(N);
         default: return false;
     }
 }
-static size_t linr_variant_shared(int v, int N) {
-    long n = v == 1 ? linr_shared_doubles<1>(N) : v == 2 ? linr_shared_doubles<2>(N)
-           : v == 3 ? linr_shared_doubles<3>(N) : linr_shared_doubles<4>(N);
-    return sizeof(double) * (size_t)n;
-}
+static size_t linr_shared(int N) { return sizeof(double) * (size_t)linr_shared_doubles(N); }
 static int linr_variant(int N) {
-    for (int v = 1; v <= 4; ++v)
+    for (int v = 1; v <= 3; ++v)
         if (linr_variant_ok(v, N)) return v;
     return 0;
 }
@@ -3444,10 +3414,10 @@ static hipError_t launch_linr(const Inst& d, int as_start, size_t shm, hipStream
     return hipGetLastError();
 }
 template <int V>
-static hipError_t launch_linr_batch(const BatchDev& b, int as_start, size_t shm, hipStream_t st) {
+static hipError_t launch_linr_batch(const BatchDev& b, int above, int upto, int as_start, size_t shm, hipStream_t st) {
     hipError_t e = allow_shared((const void*)kb_linearized<V>, shm);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((kb_linearized<V>), dim3(b.n), dim3(LinrV<V>::T), shm, st, b.inst, as_start);
+    hipLaunchKernelGGL((kb_linearized<V>), dim3(b.n), dim3(LinrV<V>::T), shm, st, b.inst, above, upto, as_start);
     return hipGetLastError();
 }
 template <int V>
@@ -3501,12 +3471,11 @@ hipError_t launch_linearized(const Inst& d, int as_start, hipStream_t st) {
     if (N < 1 || N > 1024) return hipErrorInvalidValue;
     const int v = linr_variant(N);
     if (v) {
-        const size_t shm = linr_variant_shared(v, N);
+        const size_t shm = linr_shared(N);
         switch (v) {
             case 1: return launch_linr<1>(d, as_start, shm, st);
             case 2: return launch_linr<2>(d, as_start, shm, st);
-            case 3: return launch_linr<3>(d, as_start, shm, st);
-            default: return launch_linr<4>(d, as_start, shm, st);
+            default: return launch_linr<3>(d, as_start, shm, st);
         }
     }
     if (!d.lin) return hipErrorInvalidValue;
@@ -3530,13 +3499,16 @@ hipError_t launch_linearized(const Inst& d, int as_start, hipStream_t st) {
 }
 
 hipError_t launch_gauss_dense(const double* A, const double* b, int N, double* x, int* status, int variant, hipStream_t st) {
-    if (!linr_variant_ok(variant, N)) return hipErrorInvalidValue;
-    const size_t shm = linr_variant_shared(variant, N);
-    switch (variant) {
+    // the checks' four numbers: up to 64, 127 and 128 rows, and what shared memory holds
+    const int most[] = {0, 64, 127, 128, 192};
+    if (variant < 1 || variant > 4 || N > most[variant]) return hipErrorInvalidValue;
+    const int v = variant == 1 ? 1 : variant == 4 ? 3 : 2;
+    if (!linr_variant_ok(v, N)) return hipErrorInvalidValue;
+    const size_t shm = linr_shared(N);
+    switch (v) {
         case 1: return launch_linr_dense<1>(A, b, N, x, status, shm, st);
         case 2: return launch_linr_dense<2>(A, b, N, x, status, shm, st);
-        case 3: return launch_linr_dense<3>(A, b, N, x, status, shm, st);
-        default: return launch_linr_dense<4>(A, b, N, x, status, shm, st);
+        default: return launch_linr_dense<3>(A, b, N, x, status, shm, st);
     }
 }
 
@@ -3845,20 +3817,21 @@ size_t batch_linearized_shared(const int* ns, int n, int variant) {
     size_t m = 0;
     for (int i = 0; i < n; ++i) {
         if (!linr_variant_ok(variant, ns[i])) return 0;
-        const size_t x = linr_variant_shared(variant, ns[i]);
+        const size_t x = linr_shared(ns[i]);
         m = x > m ? x : m;
     }
     return m;
 }
 
+// Systems of up to 64 rows go to workgroups of their own size: four waves and 39 KB,
+// so that four share a CU, where the largest system's workgroup takes one.
 hipError_t launch_batch_linearized(const BatchDev& b, int variant, size_t shm, int as_start, hipStream_t st) {
-    switch (variant) {
-        case 1: return launch_linr_batch<1>(b, as_start, shm, st);
-        case 2: return launch_linr_batch<2>(b, as_start, shm, st);
-        case 3: return launch_linr_batch<3>(b, as_start, shm, st);
-        case 4: return launch_linr_batch<4>(b, as_start, shm, st);
-        default: return hipErrorInvalidValue;
-    }
+    if (variant == 1) return launch_linr_batch<1>(b, 0, WAVE, as_start, shm, st);
+    hipError_t e = variant == 2   ? launch_linr_batch<2>(b, WAVE, 2 * WAVE, as_start, shm, st)
+                   : variant == 3 ? launch_linr_batch<3>(b, WAVE, 3 * WAVE, as_start, shm, st)
+                                  : hipErrorInvalidValue;
+    if (e != hipSuccess) return e;
+    return launch_linr_batch<1>(b, 0, WAVE, as_start, linr_shared(WAVE), st);
 }
 
 hipError_t launch_batch_take_singular(const BatchDev& b, double* flags, hipStream_t st) {
