@@ -1510,6 +1510,41 @@ __device__ inline V3 induced_at(const Inst& d, V3 fixed, const double* G, int i)
     return ind;
 }
 
+// induced_at of all control points by the whole workgroup, into ind [3 N] (shared): a
+// chain (point, component) per thread, so that a column's factors are read by neighbouring
+// lanes and IND_U columns are in flight per thread.  One strip's three chains per thread
+// left the loads' latency in the open: Linearized step's kernel at 120 strips 219 ->
+// 201 us.  (The fixed-point solve, whose threads' three chains overlap, lost by it: 160
+// strips 333 -> 446 us.)  Every thread calls it; ends with a barrier.
+constexpr int IND_U = 32;
+__device__ inline void induced_group(const Inst& d, const double* G, double* ind) {
+    const int N = d.N, C = 3 * N;
+    for (int ch = threadIdx.x; ch < C; ch += (int)blockDim.x) {
+        const double* F = d.F + ch;
+        double sum = 0.0;
+        int j = 0;
+        for (; j + IND_U <= N; j += IND_U) {
+            double f[IND_U];
+#pragma unroll
+            for (int u = 0; u < IND_U; ++u) f[u] = F[(long)C * (j + u)];
+#pragma unroll
+            for (int u = 0; u < IND_U; ++u) sum += f[u] * G[j + u];
+        }
+        if (j < N) {
+            double f[IND_U];
+#pragma unroll
+            for (int u = 0; u < IND_U; ++u) f[u] = F[(long)C * min(j + u, N - 1)];
+#pragma unroll
+            for (int u = 0; u < IND_U; ++u)
+                if (j + u < N) sum += f[u] * G[j + u];
+        }
+        double v = d.fixed[ch];
+        v += sum;
+        ind[ch] = v;
+    }
+    __syncthreads();
+}
+
 // velocity_corrections.rs:18-100: felt velocity plus the (corrected) induced velocity.
 __device__ inline V3 corrected_velocity(int vc_mode, double vc_ratio, V3 felt, V3 ind) {
     if (vc_mode == 1) {
@@ -1529,18 +1564,31 @@ __device__ inline double angle_of_attack(const Strip& s, V3 u) {  // force_calcu
     return len(u) > MIN_POSITIVE ? signed_angle_between(s.chord_g, u, s.dir_g) : 0.0;
 }
 
-// One evaluation of the fixed-point map for strip i from the circulations in G
-// (simple_iterative.rs:110-160): induced velocity, velocity correction,
+// One evaluation of the fixed-point map for a strip from its induced velocity
+// (simple_iterative.rs:110-160): velocity correction,
 // spanwise part removed, angle of attack, circulation estimate.
-__device__ inline double estimate_circulation(const Inst& d, const Strip& s, const double* G, int i, V3& u,
-                                              double& a) {
-    V3 ind = induced_at(d, s.fixed, G, i);
+__device__ inline double estimate_circulation(const Inst& d, const Strip& s, V3 ind, V3& u, double& a) {
     u = corrected_velocity(d.vc_mode, d.vc_ratio, s.felt, ind);
     u = u - project(u, s.rel_g);  // line_force_model/mod.rs:235-254
     a = angle_of_attack(s, u);
     return circulation(s, d.viscous_lift_in_circulation, a, u);
 }
 
+// The sum of x[0..n) in shared memory, one after another: 16 values are in flight while
+// 16 are added.
+__device__ inline double sum_in_order(const double* x, int n) {
+    double s = 0.0;
+    int q = 0;
+    for (; q + 16 <= n; q += 16) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = x[q + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += v[u];
+    }
+    for (; q < n; ++q) s += x[q];
+    return s;
+}
 __device__ inline void solve_body(const Inst& d, double* sh) {
     int N = d.N;
     double* G = sh;             // [N] current circulation (broadcast for the matvec)
@@ -1564,9 +1612,7 @@ __device__ inline void solve_body(const Inst& d, double* sh) {
     if (act) R[i] = residual_term(s, rho, g, a, u);
     __syncthreads();
     if (i == 0) {
-        double sum = 0.0;
-        for (int q = 0; q < N; ++q) sum += R[q];
-        ctl[0] = sum / (double)N;
+        ctl[0] = sum_in_order(R, N) / (double)N;
         ctl[1] = 0.0;
     }
     __syncthreads();
@@ -1579,7 +1625,7 @@ __device__ inline void solve_body(const Inst& d, double* sh) {
         __syncthreads();
         double ad = 0.0;
         if (act) {
-            est = estimate_circulation(d, s, G, i, u, a);
+            est = estimate_circulation(d, s, induced_at(d, s.fixed, G, i), u, a);
             R[i] = residual_term(s, rho, g, a, u);
             double diff = est - g;
             ad = fabs(diff);
@@ -1591,9 +1637,7 @@ __device__ inline void solve_body(const Inst& d, double* sh) {
         if ((i % WAVE) == 0) wm[i / WAVE] = m;
         __syncthreads();
         if (i == 0) {
-            double sum = 0.0;
-            for (int q = 0; q < N; ++q) sum += R[q];
-            double residual = sum / (double)N;
+            double residual = sum_in_order(R, N) / (double)N;
             double mx = 0.0;
             for (int w = 0; w < (int)((blockDim.x + WAVE - 1) / WAVE); ++w) mx = fmax_(mx, wm[w]);
             ctl[0] = residual;
@@ -1844,27 +1888,28 @@ __device__ inline void lin_outputs(const Inst& d, const Strip& s, double g, V3 u
         d.prev_gamma[t] = g;
     }
     if (t == 0) {
-        double sum = 0.0;
-        for (int q = 0; q < N; ++q) sum += R[q];
         d.out[OutLayout::iters(N, d.W)] = 1.0;
-        d.out[OutLayout::residual(N, d.W)] = sum / (double)N;
+        d.out[OutLayout::residual(N, d.W)] = sum_in_order(R, N) / (double)N;
     }
 }
-// The one-workgroup form: G holds the solution.
-__device__ inline void lin_finish(const Inst& d, const Strip& s, double* G, double* R, int as_start) {
+// The one-workgroup form: G holds the solution; ind is [3 N] shared scratch.
+__device__ inline void lin_finish(const Inst& d, const Strip& s, double* G, double* R, double* ind, int as_start) {
     const int t = threadIdx.x;
     const bool act = t < d.N;
     const int ic = act ? t : d.N - 1;
     double g = G[ic];
-    const V3 ind1 = induced_at(d, s.fixed, G, ic);
-    V3 u = lin_velocity(d, s, ind1, as_start);
+    induced_group(d, G, ind);
+    V3 u = lin_velocity(d, s, load3(ind + 3 * ic), as_start);
     if (lin_viscous(d, as_start)) {
         g = lin_viscous_gamma(s, g, u);
         __syncthreads();
         if (act) G[t] = g;
         __syncthreads();
         // NoCorrection keeps the induced velocity of the linear solution
-        u = lin_velocity(d, s, lin_second_velocity(d, as_start) ? induced_at(d, s.fixed, G, ic) : ind1, as_start);
+        if (lin_second_velocity(d, as_start)) {
+            induced_group(d, G, ind);
+            u = lin_velocity(d, s, load3(ind + 3 * ic), as_start);
+        }
     }
     lin_outputs(d, s, g, u, R, as_start);
 }
@@ -1886,7 +1931,7 @@ __device__ inline void lin_finish(const Inst& d, const Strip& s, double* G, doub
 //   - barrier.
 // Wave 0 then back-substitutes.  The pivots' chain bounds it (a pivot costs ~1,200
 // cycles; with every wave searching, the pivot row published through shared memory and
-// two barriers per pivot it was 3,300): 120 strips, kernel 271 -> 219 us (elimination 165
+// two barriers per pivot it was 3,300): 120 strips, kernel 271 -> 201 us (elimination 165
 // -> 107, back substitution 62); 1,024 instances of 8-128 strips 815 -> 600.
 constexpr int LINR_B = 8;
 template <int V>
@@ -2247,10 +2292,10 @@ __device__ inline void linearized_lds_body(const Inst& d, double* sh, int as_sta
         }
         __syncthreads();
     }
-    lin_finish(d, load_strip(d, t < N ? t : N - 1), G, R, as_start);
+    lin_finish(d, load_strip(d, t < N ? t : N - 1), G, R, sh, as_start);  // the matrix's place for ind
 }
 template <int V>
-__global__ __launch_bounds__(LinrV<V>::T) __attribute__((amdgpu_waves_per_eu(V == 1 ? 4 : 2))) void k_linearized(Inst d, int as_start) {
+__global__ __launch_bounds__(LinrV<V>::T) void k_linearized(Inst d, int as_start) {
     extern __shared__ double sh[];
     linearized_lds_body<V>(d, sh, as_start);
 }
@@ -2846,7 +2891,7 @@ __global__ void kb_horseshoe_factors(const Inst* I, const long* off, int n) {
 // One workgroup per instance (the one-workgroup Linearized form).
 // The instances with above < N <= upto.
 template <int V>
-__global__ __launch_bounds__(LinrV<V>::T) __attribute__((amdgpu_waves_per_eu(V == 1 ? 4 : 2))) void kb_linearized(const Inst* I, int above, int upto, int as_start) {
+__global__ __launch_bounds__(LinrV<V>::T) void kb_linearized(const Inst* I, int above, int upto, int as_start) {
     extern __shared__ double sh[];
     const Inst d = I[blockIdx.x];
     if (d.N <= above || d.N > upto) return;
@@ -3251,7 +3296,7 @@ __global__ __launch_bounds__(1024) void kb_warm_judge(const Inst* I, const long*
         if (act) {
             V3 u{0.0, 0.0, 0.0};
             double a = 0.0;
-            ad = fabs(estimate_circulation(d, s, G, i, u, a) - cand[c]);
+            ad = fabs(estimate_circulation(d, s, induced_at(d, s.fixed, G, i), u, a) - cand[c]);
         }
         double m = ad;
         for (int off = WAVE / 2; off > 0; off >>= 1) m = fmax_(m, __shfl_xor(m, off, WAVE));
