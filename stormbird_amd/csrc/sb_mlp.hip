@@ -427,6 +427,34 @@ __global__ void k_sum_slices(const float* part, int slices, long n, float* out) 
     out[i] = s;
 }
 
+// The same for few outputs (n up to some hundreds), where a thread per output would be a
+// few waves waiting on their loads: 16 threads per output, each a sixteenth of the slices
+// in order, their sums added in order (512 slices of the head's 257 gradients and the four layers'
+// biases, 65,536 rows: 45 -> 24 us a training step).
+__global__ __launch_bounds__(256) void k_sum_slices_few(const float* part, int slices, long n, float* out) {
+    __shared__ float sums[16][17];
+    const int c = threadIdx.x & 15, q = threadIdx.x >> 4;
+    const long i = (long)blockIdx.x * 16 + c;
+    const int per = (slices + 15) / 16, b = q * per < slices ? q * per : slices, e = b + per < slices ? b + per : slices;
+    float s = 0.f;
+    if (i < n) {
+        int k = b;
+        for (; k + 8 <= e; k += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = part[(long)(k + u) * n + i];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
+        for (; k < e; ++k) s += part[(long)k * n + i];
+    }
+    sums[q][c] = s;
+    __syncthreads();
+    if (q == 0 && i < n) {
+        for (int k = 1; k < 16; ++k) s += sums[k][c];
+        out[i] = s;
+    }
+}
 __global__ void k_to_bf16(const float* x, long n, uint16_t* y) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) y[i] = f2bf(x[i]);
@@ -464,7 +492,18 @@ __global__ void k_head_grad(const float* dy, const uint16_t* H, long n, int chun
     int k = threadIdx.x;  // 0..256 (256 = bias)
     long r0 = (long)blockIdx.x * chunk, r1 = r0 + chunk < n ? r0 + chunk : n;
     float s = 0.f;
-    for (long r = r0; r < r1; ++r) s += dy[r] * (k < 256 ? bf2f(H[r * 256 + k]) : 1.0f);
+    long r = r0;
+    for (; r + 16 <= r1; r += 16) {  // sixteen rows in flight, added in order (38 -> 33 us at 65,536 rows)
+        float h[16], e[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            h[u] = k < 256 ? bf2f(H[(r + u) * 256 + k]) : 1.0f;
+            e[u] = dy[r + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += e[u] * h[u];
+    }
+    for (; r < r1; ++r) s += dy[r] * (k < 256 ? bf2f(H[r * 256 + k]) : 1.0f);
     part[(long)blockIdx.x * 257 + k] = s;
 }
 
@@ -490,15 +529,26 @@ __global__ void k_weights_bf16(const float* W, int out, int in, uint16_t* Wb, ui
     WTb[(long)i * out + o] = h;
 }
 
-__global__ void k_reduce_sq(const float* sq, long n, float* out) {
+// Mean of sq: 256 strided sums, then those in order; 32 loads of a thread in flight
+// (one: 59 us for 65,536 rows, now 7).
+__global__ __launch_bounds__(256) void k_reduce_sq(const float* sq, long n, float* out) {
     __shared__ float red[256];
     float s = 0.f;
-    for (long i = threadIdx.x; i < n; i += 256) s += sq[i];
+    long i = threadIdx.x;
+    for (; i + 31 * 256 < n; i += 32 * 256) {
+        float v[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) v[u] = sq[i + u * 256];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) s += v[u];
+    }
+    for (; i < n; i += 256) s += sq[i];
     red[threadIdx.x] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
         float t = 0.f;
-        for (int i = 0; i < 256; ++i) t += red[i];
+#pragma unroll 32
+        for (int k = 0; k < 256; ++k) t += red[k];
         out[0] = t / (float)n;
     }
 }
@@ -651,7 +701,7 @@ struct sb_mlp {
         hipLaunchKernelGGL(k_gemm_tn, dim3(nblk(I, GT), nblk(O, GT), slices), dim3(256), 0, stream, a);
         hipLaunchKernelGGL(k_sum_slices, dim3(nblk((long)O * I, 256)), dim3(256), 0, stream, part, slices,
                            (long)O * I, C);
-        hipLaunchKernelGGL(k_sum_slices, dim3(nblk(O, 256)), dim3(256), 0, stream, a.part_bias, slices, (long)O,
+        hipLaunchKernelGGL(k_sum_slices_few, dim3(nblk(O, 16)), dim3(256), 0, stream, a.part_bias, slices, (long)O,
                            bias_grad);
         check(hipGetLastError(), "gemm");
     }
@@ -698,7 +748,7 @@ struct sb_mlp {
         // head
         ensure_part(nch * 257);
         hipLaunchKernelGGL(k_head_grad, dim3((unsigned)nch), dim3(257), 0, stream, dy, Hb[3], n, chunk, part);
-        hipLaunchKernelGGL(k_sum_slices, dim3(nblk(257, 256)), dim3(256), 0, stream, part, (int)nch, 257L,
+        hipLaunchKernelGGL(k_sum_slices_few, dim3(nblk(257, 16)), dim3(256), 0, stream, part, (int)nch, 257L,
                            g + param_offset(4));
         const float* w4 = p + param_offset(4);
         hipLaunchKernelGGL(k_head_back, dim3(nblk(n * 256, 256)), dim3(256), 0, stream, dy, w4, Z[3], n, dZb);
