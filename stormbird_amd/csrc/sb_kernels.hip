@@ -1950,7 +1950,8 @@ struct LinrV<3> {
 };
 template <int V>
 SB_HD inline bool linr_fits(int N) { return N >= 1 && N <= WAVE * LinrV<V>::RL; }
-// Shared memory (doubles): matrix [N + 1][ld], G [N] (+8), R [N], the back
+// Shared memory (doubles): matrix [N + 1][ld] (after the solve the induced velocities
+// [3 N], which are more than the matrix at N = 1), G [N] (+8), R [N], the back
 // substitution's two product rows, the rows' sources [N] (ints), the singular step.
 // Every region starts on a 16-byte boundary.
 struct LinrLayout {
@@ -1958,13 +1959,14 @@ struct LinrLayout {
     int ld;
     int pstride;  // product row stride of the back substitution
 };
-SB_HD inline long linr_even(long v) { return (v + 1) & ~1L; }
+SB_HD constexpr long linr_even(long v) { return (v + 1) & ~1L; }
 constexpr int LINR_PS = 3;  // product slots per lane of the back substitution (N <= 192)
-SB_HD inline LinrLayout linr_layout(int N) {
-    LinrLayout L;
+SB_HD constexpr LinrLayout linr_layout(int N) {
+    LinrLayout L{};
     L.ld = N | 1;
     L.pstride = (int)(N + 40 > 64 * LINR_PS ? linr_even(N + 40) : 64 * LINR_PS);
-    L.G = linr_even((long)(N + 1) * L.ld);
+    const long matrix = (long)(N + 1) * L.ld, induced = 3L * N;
+    L.G = linr_even(matrix > induced ? matrix : induced);
     L.R = L.G + linr_even(N + 8);
     L.prod = L.R + linr_even(N);
     L.src = L.prod + 2L * L.pstride + 16;
@@ -1972,6 +1974,16 @@ SB_HD inline LinrLayout linr_layout(int N) {
     return L;
 }
 SB_HD inline long linr_shared_doubles(int N) { return linr_layout(N).total; }
+constexpr bool linr_regions_apart() {
+    for (int N = 1; N <= WAVE * LINR_PS; ++N) {
+        const LinrLayout L = linr_layout(N);
+        if (L.G < (long)(N + 1) * L.ld || L.G < 3L * N || L.R < L.G + N || L.prod < L.R + N ||
+            L.src < L.prod + 2L * L.pstride || 2 * (L.total - L.src) < N + 1)
+            return false;
+    }
+    return true;
+}
+static_assert(linr_regions_apart(), "a region of the one-workgroup Linearized solve overlaps the next");
 
 template <int CTRL>
 __device__ inline double dpp_f64(double v) {

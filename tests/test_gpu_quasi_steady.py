@@ -93,6 +93,21 @@ def test_linearized_settings_in_global_memory(oracle, solver):
     run_pair(oracle, js, [6.0, 2.0, 0], steps=2)
 
 
+@pytest.mark.parametrize("nr_strips", [1, 2])
+@pytest.mark.parametrize("solver", [
+    None,
+    {"Linearized": {"induced_velocity_correction_method": "NoCorrection"}},
+    {"Linearized": {"disable_viscous_corrections": True}},
+    {"start_with_linearized_solution": True},
+])
+def test_linearized_smallest_systems(oracle, nr_strips, solver):
+    """One and two strips: the induced velocities (three per strip) in the shared memory of a matrix
+    that is smaller than they are at one strip."""
+    js = S.with_settings(S.rectangular_wing(aspect_ratio=3.0, cl_zero_angle=0.3, angle_of_attack=4 * S.DEG,
+                                            nr_strips=nr_strips), S.quasi_steady_settings(solver=solver))
+    run_pair(oracle, js, [7.0, 0.5, 0], steps=3)
+
+
 def test_quasi_steady_simple_iterative_and_linearized_start(oracle):
     base = {"max_iterations_per_time_step": 3000, "residual_tolerance_absolute": 1e-9,
             "strength_difference_tolerance": 1e-10}
