@@ -2662,9 +2662,19 @@ __global__ void k_gauss_status(Inst d, int* status) { *status = (int)d.scal[4]; 
 // flow_derivatives.rs:31-62), one workgroup
 // ---------------------------------------------------------------------------
 constexpr int FORCE_CHUNK = 64;
+constexpr int FORCE_WINGS = 1024;  // wings whose strips are looked up in shared memory
+__device__ inline int first_strip(const int* wing_of, int N, int w) {  // of wing w or behind it (wing_of ascends)
+    int a = 0, b = N;
+    while (a < b) {
+        const int m = (a + b) / 2;
+        if (wing_of[m] < w) a = m + 1;
+        else b = m;
+    }
+    return a;
+}
 __device__ inline void forces_body(const Inst& d, double dt) {
     __shared__ double terms[36][FORCE_CHUNK + 1];  // rows start in different banks
-    __shared__ int wing_lo[1024], wing_hi[1024];   // strips of each wing
+    __shared__ int wing_lo[FORCE_WINGS], wing_hi[FORCE_WINGS];  // strips of each wing
     int N = d.N, W = d.W;
     const double* geo = d.geo;
     double* o = d.out;
@@ -2744,7 +2754,12 @@ __device__ inline void forces_body(const Inst& d, double dt) {
     // 32 us, 3 x 40: 22.5 -> 8.6, 20: 12.4 -> 7.8).
     const bool real = i < N && geo[d.gl.is_virtual + i] == 0.0;
     const V3 arm = i < N ? load3(geo + d.gl.ctrl_out + 3 * i) : V3{0.0, 0.0, 0.0};
-    if (i < N) {
+    // A wing of zero length has no strips: its range stays empty, its sums +0.  (With such
+    // wings there may be more wings than strips, and more than the arrays hold.)
+    const bool listed = W <= FORCE_WINGS;
+    for (int w = i; listed && w < W; w += (int)blockDim.x) wing_lo[w] = wing_hi[w] = 0;
+    __syncthreads();
+    if (listed && i < N) {
         const int w = d.wing_of[i];
         if (i == 0 || d.wing_of[i - 1] != w) wing_lo[w] = i;
         if (i == N - 1 || d.wing_of[i + 1] != w) wing_hi[w] = i + 1;
@@ -2770,8 +2785,10 @@ __device__ inline void forces_body(const Inst& d, double dt) {
             }
             __syncthreads();
             if (idx < sums) {
-                const int lo = wing_lo[w] > q0 ? wing_lo[w] - q0 : 0;
-                const int hi = wing_hi[w] < q0 + FORCE_CHUNK ? wing_hi[w] - q0 : FORCE_CHUNK;
+                const int first = listed ? wing_lo[w] : first_strip(d.wing_of, N, w);
+                const int end = listed ? wing_hi[w] : first_strip(d.wing_of, N, w + 1);
+                const int lo = first > q0 ? first - q0 : 0;
+                const int hi = end < q0 + FORCE_CHUNK ? end - q0 : FORCE_CHUNK;
                 int q = lo;
                 for (; q + 8 <= hi; q += 8) {
                     double v[8];

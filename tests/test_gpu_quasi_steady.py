@@ -108,6 +108,37 @@ def test_linearized_smallest_systems(oracle, nr_strips, solver):
     run_pair(oracle, js, [7.0, 0.5, 0], steps=3)
 
 
+@pytest.mark.parametrize("empty", [1, 1100])
+def test_integrated_forces_of_wings_without_strips(empty):
+    """Wings of zero length are cut into no strips: their integrated forces and moments are zero, and the
+    other wings' equal those of the setup without them, alone and in a batch (1,100: more wings than strips)."""
+    d = json.loads(S.wing_sails_quasi_steady(nr_strips=5))
+    wings = d["line_force_model"]["wing_builders"][:2]
+    point = json.loads(json.dumps(wings[0]))
+    point["section_points"][1] = dict(point["section_points"][0])
+
+    def make(builders):
+        d["line_force_model"]["wing_builders"] = builders
+        return json.dumps(d)
+
+    plain, holed = make(wings), make([wings[0]] + [point] * empty + [wings[1]])
+    a, b = sb.Simulation(plain), sb.Simulation(holed)
+    both = sb.Batch([holed, plain])
+    fs = S.uniform_freestream(a.nr_freestream_points(), [6.0, 2.0, 0.0])
+    assert b.nr_freestream_points() == a.nr_freestream_points() == 10
+    for k in range(3):
+        ra = a.do_step(time=k * 1.0, time_step=1.0, freestream_velocity=fs).as_arrays()
+        results = both.do_step(times=k * 1.0, time_steps=1.0, freestream_velocity=np.concatenate([fs, fs]))
+        for rb in (b.do_step(time=k * 1.0, time_step=1.0, freestream_velocity=fs), results[0]):
+            rb = rb.as_arrays()
+            for key in ("circulation_strength", "sectional_forces"):
+                assert same(rb[key], ra[key]), key
+            for key in ("integrated_forces", "integrated_moments"):
+                sums = rb[key].reshape(6, 2 + empty, 3)
+                assert same(sums[:, [0, -1]], ra[key].reshape(6, 2, 3)), key
+                assert not sums[:, 1:-1].any(), key
+
+
 def test_quasi_steady_simple_iterative_and_linearized_start(oracle):
     base = {"max_iterations_per_time_step": 3000, "residual_tolerance_absolute": 1e-9,
             "strength_difference_tolerance": 1e-10}
