@@ -216,6 +216,7 @@ struct sb_batch {
         bd.max_threads = std::min(1024, ((max_n + 63) / 64) * 64);
         bd.solve_shm = solve_shared_bytes(max_n, max_w);
         bd.counters = d_counters;
+        check(hipDeviceGetAttribute(&bd.cus, hipDeviceAttributeMultiprocessorCount, device), "device attribute");
         bd.sym = sym;
         bd.stage_near = 1;
         for (auto& s : sims)
@@ -363,6 +364,7 @@ struct sb_batch {
         }
         bd.n_fixed_jobs = (int)fj.size();
         bd.n_target_jobs = (int)nt;
+        bd.targets_few = batch_targets_few(mode, bd.cus, nt);
         fixed_work = 0.0;
         for (const auto& f : fj) fixed_work += (double)FIXED_JOB_TARGETS * (double)f.first;
         target_work = 0.0;
@@ -391,7 +393,7 @@ struct sb_batch {
         const bool apply = mlp && (when >= 2 || (when == 1 && first));
         const bool feats = apply || record_features;
         last_applied = apply;
-        long sig[3] = {first ? 1 : 0, bd.n_fixed_jobs, (bd.n_target_jobs * 8 + (apply ? warm_mode : 0)) * 2 + (feats ? 1 : 0)};
+        long sig[3] = {first ? 1 : 0, bd.n_fixed_jobs * 2L + bd.targets_few, (bd.n_target_jobs * 8 + (apply ? warm_mode : 0)) * 2 + (feats ? 1 : 0)};
         if (first || !use_graph) {
             enqueue(first, apply, feats);
         } else {
@@ -520,7 +522,9 @@ struct sb_batch {
 
     // Key of the tuning cache: the device, the arithmetic, and the shape class of the
     // last step's work (powers of two of the instance count and of both pair sums, the
-    // largest strip count in units of 64).
+    // largest strip count in units of 64, the self-induction kernel).  The number behind
+    // "kernels" grows when a tuned parameter comes to mean something else, so that a
+    // choice made for other kernels is not applied.
     std::string tuning_key() const {
         hipDeviceProp_t prop;
         check(hipGetDeviceProperties(&prop, device), "device properties");
@@ -530,14 +534,15 @@ struct sb_batch {
         std::ostringstream k;
         k << prop.gcnArchName << "|" << prop.name << "|" << (mode == MODE_FAST ? "fast" : "exact") << "|sym"
           << bd.sym << "|n" << lg((double)n) << "|f" << lg(fixed_work) << "|t" << lg(target_work) << "|N"
-          << (max_n + 63) / 64;
+          << (max_n + 63) / 64 << "|few" << bd.targets_few << "|kernels3";
         return k.str();
     }
 
     // Times every variant of the batched pair kernels on the batch's own last-step state
     // (outputs saved and restored, so the state is unchanged) and applies the fastest.
     // timings: kb_fixed for 1, 2, 3 fours of panels per wave, then kb_targets for 64, 128, 256
-    // records per tile (ms, -1 where a kernel had no work).
+    // records per tile (ms, -1 where a kernel had no work).  The few-target self-induction
+    // kernel has no tile: it is timed once, for all three, and the tile stays.
     void autotune(double* timings, int reps, long max_jobs) {
         if (quasi) throw std::invalid_argument("the autotuner covers dynamic batches");
         if (!first_done) throw std::invalid_argument("take a step before tuning: the jobs come from the last step");
@@ -602,15 +607,15 @@ struct sb_batch {
                 if (timings) timings[v] = t;
             }
             tbest = 1e300;
+            double t = -1.0;
             for (int v = 0; v < 3; ++v) {
-                double t = -1.0;
-                if (targets) {
-                    set_tuning(best_per, tiles[v]);
+                if (targets && !(v > 0 && bd.targets_few)) {
+                    set_tuning(best_per, bd.targets_few ? prev_tile : tiles[v]);
                     BatchDev b = bd;
                     b.inst = d_inst + 3L * n;
                     if (max_jobs > 0 && b.n_target_jobs > max_jobs) b.n_target_jobs = (int)max_jobs;
                     t = time_launch([&] { check(launch_batch_self_induction(b, mode, stream), "self induction"); });
-                    if (t < tbest) {
+                    if (t < tbest && !bd.targets_few) {
                         tbest = t;
                         best_tile = tiles[v];
                     }
@@ -752,6 +757,8 @@ int sb_batch_get_tuning(const sb_batch* b, int* fixed_per, int* targets_tile) {
     *targets_tile = b->bd.targets_tile;
     return 0;
 }
+
+int sb_debug_batch_targets_few(const sb_batch* b) { return b ? b->bd.targets_few : -1; }
 
 int sb_batch_autotune(sb_batch* b, const char* cache_path, int flags, int reps, long max_jobs, double* timings,
                       size_t cap) {

@@ -228,6 +228,8 @@ struct BatchDev {
     int fixed_grid = 0, target_grid = 0;  // persistent workgroups
     int fixed_per = 3;            // kb_fixed: fours of panels per compute wave per block (1, 2, 3)
     int targets_tile = 256;       // kb_targets: panel records per LDS tile (64, 128, 256)
+    int cus = 0;                  // compute units of the batch's device
+    int targets_few = 0;          // self-induction: 1 for kb_targets_few (batch_targets_few on the whole queue)
     int stage_near = 0;           // kb_targets: 1 when every self-induced instance has ring-edge
                                   // geometry (near-field data staged with the records)
     int sym = 0;                  // 1 when any instance uses a symmetry plane
@@ -251,6 +253,8 @@ hipError_t launch_batch_factors(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_solve(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_velocity_copy(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_self_induction(const BatchDev& b, int mode, hipStream_t st);
+// Whether a batch of n_jobs target jobs takes kb_targets_few (16 wake points per workgroup).
+bool batch_targets_few(int mode, int cus, long n_jobs);
 hipError_t launch_batch_forces(const BatchDev& b, hipStream_t st);
 // Features of every strip (kb_features) and, when `apply` is 1, the network's
 // initial circulation written into prev_gamma (after the prepare kernel); with

@@ -3925,6 +3925,11 @@ hipError_t launch_batch_velocity_copy(const BatchDev& b, hipStream_t st) {
     return hipGetLastError();
 }
 
+// few: up to 3 workgroups of 256 per CU in EXACT (12 ships, 936 of them: 50.6 ms per
+// step against 50.0; 8 ships, 624: 34.2 against 42.7; 4: 17.9 against 30.0), up to 1.5
+// in FAST, whose sweep gains more from the wave-uniform panel
+bool batch_targets_few(int mode, int cus, long n_jobs) { return 2 * n_jobs <= (mode == MODE_EXACT ? 6 : 3) * (long)cus; }
+
 template <int MODE, int SYM, int TL>
 static void launch_kb_targets(const BatchDev& b, hipStream_t st) {
     if (b.stage_near)
@@ -3937,11 +3942,8 @@ static void launch_kb_targets(const BatchDev& b, hipStream_t st) {
 
 template <int MODE, int SYM>
 static void launch_kb_targets_tile(const BatchDev& b, hipStream_t st) {
-    // few: up to 3 workgroups of 256 per CU in EXACT (12 ships, 936 of them: 50.6 ms per
-    // step against 50.0; 8 ships, 624: 34.2 against 42.7; 4: 17.9 against 30.0), up to 1.5
-    // in FAST, whose sweep gains more from the wave-uniform panel
-    if (2 * b.n_target_jobs <= (MODE == MODE_EXACT ? 6 : 3) * cu_count()) {
-        hipLaunchKernelGGL((kb_targets_few<MODE, SYM>), dim3((unsigned)cu_count()), dim3(FX_WAVES * WAVE), 0, st, b.inst,
+    if (b.targets_few) {
+        hipLaunchKernelGGL((kb_targets_few<MODE, SYM>), dim3((unsigned)b.cus), dim3(FX_WAVES * WAVE), 0, st, b.inst,
                            b.target_jobs, b.n_target_jobs, b.counters + 1);
         return;
     }

@@ -313,3 +313,64 @@ def test_residual_warm_start_with_a_zero_network_is_the_default_guess():
         for i in range(3):
             compare_results(rb[i], ra[i], exact=True, where=f"step {k} ship {i}")
     assert b.batch.last_fallbacks() == 0
+
+
+def few_route(batch):
+    """1 when the batch's last self-induction took the kernel for few wake points, else 0."""
+    import ctypes
+
+    L = sb.lib()
+    L.sb_debug_batch_targets_few.argtypes = [ctypes.c_void_p]
+    return L.sb_debug_batch_targets_few(batch._h)
+
+
+def free_wake_batch(copies, rows, strips, mode, symmetry=None):
+    """`copies` of a four-sail free wake, every row shed (the initial straight wake, its strengths decaying
+    downstream), after one step with self-induction; (batch, step)."""
+    import json
+
+    js, case = S.four_sail_free_wake(nr_panels=rows, nr_strips=strips)
+    d = json.loads(js)
+    if symmetry:
+        d["simulation_settings"]["Dynamic"]["wake"]["symmetry_condition"] = symmetry
+    batch = sb.Batch([json.dumps(d)] * copies, mode=mode)
+    fs = np.tile(np.asarray(case["velocity"]), (batch.nr_freestream_points, 1))
+
+    def step():
+        return batch.do_step(times=0.0, time_steps=0.2, freestream_velocity=fs)
+
+    step()
+    n = 4 * strips
+    for i, sim in enumerate(batch.instances):
+        w = sim.get_wake_state()
+        rng = np.random.default_rng(i)
+        g = -40.0 * np.exp(-np.arange(rows) / rows)[:, None] * rng.uniform(0.5, 1.0, (rows, n))
+        p = w["points"] + rng.normal(0.0, 0.05, w["points"].shape)
+        sim.set_wake_state(p, w["velocities"], g.ravel(), rows)
+        sim.previous_circulation_strength = g[0]
+    step()
+    return batch, step
+
+
+def test_autotuner_keeps_the_self_induction_kernels_apart(tmp_path):
+    """The kernel for few wake points has no tile: one time for all three, and the tile stays.  Batches of
+    one size class (2 and 3 instances, equal powers of two of both pair counts) on the two sides of the
+    rule don't share a cache entry, and a limit on the timed jobs does not change the kernel."""
+    import json
+
+    cache = str(tmp_path / "tuning.json")
+    few, _ = free_wake_batch(2, 271, 32, sb.MODE_FAST)   # 282 workgroups of 256 on 256 CUs
+    many, step = free_wake_batch(3, 271, 32, sb.MODE_FAST)  # 423
+    assert few_route(few) == 1 and few_route(many) == 0
+    few.set_tuning(2, 128)
+    cached, choice, t = few.autotune(cache)
+    assert not cached and choice[1] == 128 and np.all(t > 0.0)
+    assert t[3] == t[4] == t[5]
+    cached, choice, t = many.autotune(cache, max_jobs=200)
+    assert not cached and np.all(t > 0.0) and len(set(t[3:])) > 1
+    assert few_route(many) == 0
+    step()
+    assert few_route(many) == 0
+    entries = json.load(open(cache))["entries"]
+    assert len(entries) == 2 and [e["targets_tile"] for e in entries] == [128, choice[1]]
+    assert len({e["key"].replace("|few1", "|few0") for e in entries}) == 1  # one size class otherwise
