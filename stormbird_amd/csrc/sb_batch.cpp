@@ -364,7 +364,6 @@ struct sb_batch {
         }
         bd.n_fixed_jobs = (int)fj.size();
         bd.n_target_jobs = (int)nt;
-        bd.targets_few = batch_targets_few(mode, bd.cus, nt);
         fixed_work = 0.0;
         for (const auto& f : fj) fixed_work += (double)FIXED_JOB_TARGETS * (double)f.first;
         target_work = 0.0;
@@ -372,6 +371,7 @@ struct sb_batch {
             const Inst& d = h_inst[3 * n + h_jobs[cap_fixed_jobs + k].x];
             target_work += 256.0 * (double)d.N * (double)d.nz_rows;
         }
+        bd.targets_few = nt > 0 && batch_targets_few(mode, bd.sym, bd.cus, nt, target_work / (256.0 * (double)nt));
 
         // freestream into the slab (outside the graph: the caller's pointer may change)
         if (wind) {

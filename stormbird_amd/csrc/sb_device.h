@@ -253,8 +253,9 @@ hipError_t launch_batch_factors(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_solve(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_velocity_copy(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_self_induction(const BatchDev& b, int mode, hipStream_t st);
-// Whether a batch of n_jobs target jobs takes kb_targets_few (16 wake points per workgroup).
-bool batch_targets_few(int mode, int cus, long n_jobs);
+// Whether a batch of n_jobs target jobs with `panels` panels each on average takes
+// kb_targets_few (16 wake points per workgroup).
+bool batch_targets_few(int mode, int sym, int cus, long n_jobs, double panels);
 hipError_t launch_batch_forces(const BatchDev& b, hipStream_t st);
 // Features of every strip (kb_features) and, when `apply` is 1, the network's
 // initial circulation written into prev_gamma (after the prepare kernel); with

@@ -3925,10 +3925,23 @@ hipError_t launch_batch_velocity_copy(const BatchDev& b, hipStream_t st) {
     return hipGetLastError();
 }
 
-// few: up to 3 workgroups of 256 per CU in EXACT (12 ships, 936 of them: 50.6 ms per
-// step against 50.0; 8 ships, 624: 34.2 against 42.7; 4: 17.9 against 30.0), up to 1.5
-// in FAST, whose sweep gains more from the wave-uniform panel
-bool batch_targets_few(int mode, int cus, long n_jobs) { return 2 * n_jobs <= (mode == MODE_EXACT ? 6 : 3) * (long)cus; }
+// The few-point kernel's time goes with the jobs, the 256-point kernel's is that of its
+// longest workgroups while every CU has at most one or two, so up to a number of jobs per
+// CU the first is faster (kernel ms few / 256-point, tile 256, at workgroups of 256 on 256
+// CUs):
+//   EXACT           624: 15.2 / 16.6, 702: 17.1 / 16.9, 758: 113 / 116        -> 3 per CU
+//   EXACT, symmetry 266: 11.1 / 11.7, 297: 8.9 / 9.6, 312: 25.1 / 23.4, 624: 49.8 / 32.5 -> 19/16
+//   FAST            312: 6.65 / 7.92, 379: 47.2 / 50.2, 390 extrapolated: 8.3 / 7.9 -> 24/16
+//   FAST, symmetry  156: 13.4 / 15.3, 161: 31.1 / 34.5, 204: 15.1 / 13.3, 312: 26.7 / 16.2 -> 11/16
+// (FAST gains more from the 256-point kernel's wave-uniform panel, and so does the mirrored
+// evaluation.)  And it works through whole blocks of 180 panels, so that few panels (the
+// first steps after the start) don't pay with many points:
+//   EXACT           145,000 points: 40 panels 0.210 / 0.145, 56: 0.205 / 0.197, 72: 0.206 / 0.225; 72,000: 40: 0.109 / 0.132
+//   EXACT, symmetry 72,000 points: 40 panels 0.33 / 0.18, 72: 0.33 / 0.29; 63,000: 100: 0.30 / 0.35
+bool batch_targets_few(int mode, int sym, int cus, long n_jobs, double panels) {
+    const long limit = mode == MODE_EXACT ? (sym ? 19 : 48) : (sym ? 11 : 24);
+    return 16 * n_jobs <= limit * cus && 256.0 * (double)n_jobs <= (sym ? 850.0 : 2500.0) * panels;
+}
 
 template <int MODE, int SYM, int TL>
 static void launch_kb_targets(const BatchDev& b, hipStream_t st) {

@@ -324,32 +324,98 @@ def few_route(batch):
     return L.sb_debug_batch_targets_few(batch._h)
 
 
-def free_wake_batch(copies, rows, strips, mode, symmetry=None):
-    """`copies` of a four-sail free wake, every row shed (the initial straight wake, its strengths decaying
-    downstream), after one step with self-induction; (batch, step)."""
+def free_wake_setup(rows, strips, symmetry=None):
     import json
 
     js, case = S.four_sail_free_wake(nr_panels=rows, nr_strips=strips)
     d = json.loads(js)
     if symmetry:
         d["simulation_settings"]["Dynamic"]["wake"]["symmetry_condition"] = symmetry
-    batch = sb.Batch([json.dumps(d)] * copies, mode=mode)
-    fs = np.tile(np.asarray(case["velocity"]), (batch.nr_freestream_points, 1))
+    return json.dumps(d), np.asarray(case["velocity"])
+
+
+def shed_every_row(sim, rows, strips, seed):
+    """A stepped simulation's straight wake with noise, every row shed, strengths decaying downstream."""
+    rng = np.random.default_rng(seed)
+    w = sim.get_wake_state()
+    g = -40.0 * np.exp(-np.arange(rows) / rows)[:, None] * rng.uniform(0.5, 1.0, (rows, 4 * strips))
+    sim.set_wake_state(w["points"] + rng.normal(0.0, 0.05, w["points"].shape), w["velocities"], g.ravel(), rows)
+    sim.previous_circulation_strength = g[0]
+
+
+def free_wake_batch(copies, rows, strips, mode, symmetry=None):
+    """`copies` of a four-sail free wake with every row shed, after one step with self-induction;
+    (batch, step)."""
+    js, u = free_wake_setup(rows, strips, symmetry)
+    batch = sb.Batch([js] * copies, mode=mode)
+    fs = np.tile(u, (batch.nr_freestream_points, 1))
 
     def step():
         return batch.do_step(times=0.0, time_steps=0.2, freestream_velocity=fs)
 
     step()
-    n = 4 * strips
     for i, sim in enumerate(batch.instances):
-        w = sim.get_wake_state()
-        rng = np.random.default_rng(i)
-        g = -40.0 * np.exp(-np.arange(rows) / rows)[:, None] * rng.uniform(0.5, 1.0, (rows, n))
-        p = w["points"] + rng.normal(0.0, 0.05, w["points"].shape)
-        sim.set_wake_state(p, w["velocities"], g.ravel(), rows)
-        sim.previous_circulation_strength = g[0]
+        shed_every_row(sim, rows, strips, i)
     step()
     return batch, step
+
+
+@pytest.mark.parametrize("symmetry", [None, "Z"])
+@pytest.mark.parametrize("mode", [sb.MODE_EXACT, sb.MODE_FAST])
+def test_every_self_induction_kernel_gives_the_same_bits(mode, symmetry):
+    """A wake of 141 workgroups of 256 points on the kernel for few points (alone and in a batch), on the
+    256-point kernel of single instances (a target map keeps it there) and on the batched 256-point
+    kernel with each tile (seven copies), with and without a symmetry plane: equal wakes."""
+    rows, strips = 271, 32
+    js, u = free_wake_setup(rows, strips, symmetry)
+    alone, tiled = sb.Simulation(js, mode=mode), sb.Simulation(js, mode=mode)
+    tiled.target_tiling = 8
+    fs = np.tile(u, (alone.nr_freestream_points(), 1))
+    few, step_few = free_wake_batch(1, rows, strips, mode, symmetry)
+    many, step_many = free_wake_batch(7, rows, strips, mode, symmetry)
+    assert few_route(few) == 1 and few_route(many) == 0
+    for sim in (alone, tiled):
+        sim.do_step(time=0.0, time_step=0.2, freestream_velocity=fs)
+        shed_every_row(sim, rows, strips, 0)
+        sim.do_step(time=0.0, time_step=0.2, freestream_velocity=fs)
+    for tile in (256, 64, 128):
+        want = alone.get_wake_state()
+        for where, sim in (("tiled", tiled), ("few", few.instances[0]), ("many", many.instances[0])):
+            got = sim.get_wake_state()
+            for key in ("points", "velocities", "strengths"):
+                assert same(got[key], want[key]), f"{where}, tile before {tile}: wake {key}"
+        many.set_tuning(3, tile)
+        step_many()
+        step_few()
+        for sim in (alone, tiled):
+            sim.do_step(time=0.0, time_step=0.2, freestream_velocity=fs)
+    want, got = alone.get_wake_state(), many.instances[0].get_wake_state()
+    for key in ("points", "velocities", "strengths"):
+        assert same(got[key], want[key]), f"tile 128: wake {key}"
+
+
+@pytest.mark.parametrize("mode,symmetry,copies,few", [
+    (sb.MODE_EXACT, None, 5, 1), (sb.MODE_EXACT, None, 6, 0),   # 705 and 846 workgroups of 256; 768 of 256 CUs
+    (sb.MODE_EXACT, "Z", 2, 1), (sb.MODE_EXACT, "Z", 3, 0),     # 282 and 423; 304
+    (sb.MODE_FAST, None, 2, 1), (sb.MODE_FAST, None, 3, 0),     # 282 and 423; 384
+    (sb.MODE_FAST, "Z", 1, 1), (sb.MODE_FAST, "Z", 2, 0),       # 141 and 282; 176
+])
+def test_self_induction_kernel_of_a_batch(mode, symmetry, copies, few):
+    """The rule between the two kernels on both sides of its measured lines: by the workgroups, and by the
+    panels in the first steps, where the wake has many points and few shed rows."""
+    import json
+
+    batch, _ = free_wake_batch(copies, 271, 32, mode, symmetry)
+    assert few_route(batch) == few
+    if mode != sb.MODE_EXACT:
+        return
+    d = json.loads(free_wake_setup(2000, 8, symmetry)[0])
+    d["line_force_model"]["wing_builders"] = d["line_force_model"]["wing_builders"][:1]
+    start = sb.Batch([json.dumps(d)] * (4 if symmetry else 8), mode=mode)  # 71 workgroups of 256 points each
+    fs = np.tile([10.0, 3.0, 0.0], (start.nr_freestream_points, 1))
+    for k in range(5):  # 40 panels
+        start.do_step(times=0.2 * k, time_steps=0.2, freestream_velocity=fs)
+    assert few_route(start) == 0
 
 
 def test_autotuner_keeps_the_self_induction_kernels_apart(tmp_path):
