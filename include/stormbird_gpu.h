@@ -339,16 +339,20 @@ int sb_batch_get_tuning(const sb_batch* b, int* fixed_per, int* targets_tile);
  * have been taken; the state is left unchanged) and applies the fastest.
  * flags bit 0: use a choice stored in cache_path for the same device and shape
  * class (instance count, pair counts and largest strip count, in powers of
- * two, and the self-induction kernel) without timing; bit 1: store the result in cache_path (a JSON file).
+ * two, and the kernels they choose) without timing; bit 1: store the result in cache_path (a JSON file).
  * Each variant runs once untimed, then `reps` timed launches (the fastest
  * counts); max_jobs > 0 times only the first max_jobs jobs of each kernel's
  * queue (the fixed-velocity queue is longest first).  timings [6] (may be
- * NULL): ms of the fixed-velocity kernel for 1, 2, 3 panels per wave, then of
- * the self-induction kernel for tiles of 64, 128, 256 (-1: no work; a batch
- * with few wake points takes a kernel without tiles: one time for all three, and
- * the tile stays).  Returns 1 when the choice came from the cache, 0 when timed. */
+ * NULL): ms of the fixed-velocity kernel for 1, 2, 3 fours of panels per wave, then
+ * of the self-induction kernel for tiles of 64, 128, 256 (-1: no work).  A batch
+ * with much fixed-velocity work (64 control points per job), or with few wake
+ * points, takes a kernel without variants: one time for all three, and the
+ * parameter stays.  Returns 1 when the choice came from the cache, 0 when timed. */
 int sb_batch_autotune(sb_batch* b, const char* cache_path, int flags, int reps, long max_jobs, double* timings,
                       size_t cap);
+/* 1 when the last dynamic step's fixed velocities took the kernel with 64 control points
+ * per job, 0 when 16, -1 for NULL. */
+int sb_debug_batch_fixed_wide(const sb_batch* b);
 /* 1 when the last dynamic step's self-induction took the kernel for few wake points
  * (16 per workgroup), 0 when 256 per workgroup, -1 for NULL. */
 int sb_debug_batch_targets_few(const sb_batch* b);

@@ -154,6 +154,7 @@ pub mod ffi {
         pub fn sb_batch_get_freestream(b: *const sb_batch, out: *mut f64, n_points: usize) -> c_int;
         pub fn sb_batch_set_tuning(b: *mut sb_batch, fixed_per: c_int, targets_tile: c_int) -> c_int;
         pub fn sb_batch_get_tuning(b: *const sb_batch, fixed_per: *mut c_int, targets_tile: *mut c_int) -> c_int;
+        pub fn sb_debug_batch_fixed_wide(b: *const sb_batch) -> c_int;
         pub fn sb_debug_batch_targets_few(b: *const sb_batch) -> c_int;
         pub fn sb_batch_autotune(b: *mut sb_batch, cache_path: *const c_char, flags: c_int, reps: c_int, max_jobs: c_long, timings: *mut f64, cap: usize) -> c_int;
         pub fn sb_mlp_create(device: c_int, seed: u64) -> *mut sb_mlp;

@@ -344,13 +344,23 @@ struct sb_batch {
             h_inst[3 * n + i] = stage_inst(i, dts[i]);
         }
         // pair-sum jobs: fixed velocities longest first; self-induction where it runs
+        double longest = 0.0, work = 0.0, work_wide = 0.0;
+        for (int i = 0; i < n; ++i) {
+            const Inst& d = h_inst[2 * n + i];
+            const double len = (double)d.N * (double)std::max(d.nz_rows - 1, 0);
+            longest = std::max(longest, len);
+            work += len * (double)((d.N + FIXED_JOB_TARGETS - 1) / FIXED_JOB_TARGETS);
+            work_wide += len * (double)((d.N + FIXED_WIDE_TARGETS - 1) / FIXED_WIDE_TARGETS);
+        }
+        bd.fixed_wide = batch_fixed_wide(mode, bd.sym, bd.cus, longest, work, work_wide);
+        const int per_job = bd.fixed_wide ? FIXED_WIDE_TARGETS : FIXED_JOB_TARGETS;
         std::vector<std::pair<long, int2>> fj;
         fj.reserve(cap_fixed_jobs);
         long nt = 0;
         for (int i = 0; i < n; ++i) {
             const Inst& d = h_inst[2 * n + i];
             long len = (long)d.N * std::max(d.nz_rows - 1, 0);
-            for (int tb = 0; tb < (d.N + FIXED_JOB_TARGETS - 1) / FIXED_JOB_TARGETS; ++tb) fj.push_back({len, int2{i, tb}});
+            for (int tb = 0; tb < (d.N + per_job - 1) / per_job; ++tb) fj.push_back({len, int2{i, tb}});
         }
         std::stable_sort(fj.begin(), fj.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
         for (size_t k = 0; k < fj.size(); ++k) h_jobs[k] = fj[k].second;
@@ -365,7 +375,7 @@ struct sb_batch {
         bd.n_fixed_jobs = (int)fj.size();
         bd.n_target_jobs = (int)nt;
         fixed_work = 0.0;
-        for (const auto& f : fj) fixed_work += (double)FIXED_JOB_TARGETS * (double)f.first;
+        for (const auto& f : fj) fixed_work += (double)per_job * (double)f.first;
         target_work = 0.0;
         for (long k = 0; k < nt; ++k) {
             const Inst& d = h_inst[3 * n + h_jobs[cap_fixed_jobs + k].x];
@@ -393,7 +403,7 @@ struct sb_batch {
         const bool apply = mlp && (when >= 2 || (when == 1 && first));
         const bool feats = apply || record_features;
         last_applied = apply;
-        long sig[3] = {first ? 1 : 0, bd.n_fixed_jobs * 2L + bd.targets_few, (bd.n_target_jobs * 8 + (apply ? warm_mode : 0)) * 2 + (feats ? 1 : 0)};
+        long sig[3] = {first ? 1 : 0, (bd.n_fixed_jobs * 2L + bd.fixed_wide) * 2L + bd.targets_few, (bd.n_target_jobs * 8 + (apply ? warm_mode : 0)) * 2 + (feats ? 1 : 0)};
         if (first || !use_graph) {
             enqueue(first, apply, feats);
         } else {
@@ -508,10 +518,12 @@ struct sb_batch {
         check(hipSetDevice(device), "hipSetDevice");
         int fg = batch_resident_groups(0, mode, bd.sym, fixed_per, 0);
         int tg = batch_resident_groups(1, mode, bd.sym, targets_tile, bd.stage_near);
-        if (fg <= 0 || tg <= 0) throw HipError("occupancy query failed", -1);
+        int wg = batch_resident_groups(2, mode, bd.sym, 0, 0);
+        if (fg <= 0 || tg <= 0 || wg <= 0) throw HipError("occupancy query failed", -1);
         bd.fixed_per = fixed_per;
         bd.targets_tile = targets_tile;
         bd.fixed_grid = fg;
+        bd.fixed_wide_grid = wg;
         bd.target_grid = tg;
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
@@ -522,7 +534,7 @@ struct sb_batch {
 
     // Key of the tuning cache: the device, the arithmetic, and the shape class of the
     // last step's work (powers of two of the instance count and of both pair sums, the
-    // largest strip count in units of 64, the self-induction kernel).  The number behind
+    // largest strip count in units of 64, the kernels).  The number behind
     // "kernels" grows when a tuned parameter comes to mean something else, so that a
     // choice made for other kernels is not applied.
     std::string tuning_key() const {
@@ -534,15 +546,16 @@ struct sb_batch {
         std::ostringstream k;
         k << prop.gcnArchName << "|" << prop.name << "|" << (mode == MODE_FAST ? "fast" : "exact") << "|sym"
           << bd.sym << "|n" << lg((double)n) << "|f" << lg(fixed_work) << "|t" << lg(target_work) << "|N"
-          << (max_n + 63) / 64 << "|few" << bd.targets_few << "|kernels3";
+          << (max_n + 63) / 64 << "|wide" << bd.fixed_wide << "|few" << bd.targets_few << "|kernels3";
         return k.str();
     }
 
     // Times every variant of the batched pair kernels on the batch's own last-step state
     // (outputs saved and restored, so the state is unchanged) and applies the fastest.
     // timings: kb_fixed for 1, 2, 3 fours of panels per wave, then kb_targets for 64, 128, 256
-    // records per tile (ms, -1 where a kernel had no work).  The few-target self-induction
-    // kernel has no tile: it is timed once, for all three, and the tile stays.
+    // records per tile (ms, -1 where a kernel had no work).  The wide fixed-velocity
+    // kernel and the few-target self-induction kernel have no variants: each is timed once,
+    // for all three, and the parameter stays.
     void autotune(double* timings, int reps, long max_jobs) {
         if (quasi) throw std::invalid_argument("the autotuner covers dynamic batches");
         if (!first_done) throw std::invalid_argument("take a step before tuning: the jobs come from the last step");
@@ -590,16 +603,15 @@ struct sb_batch {
                 return best;
             };
             const int pers[3] = {1, 2, 3}, tiles[3] = {64, 128, 256};
-            double tbest = 1e300;
+            double tbest = 1e300, t = -1.0;
             for (int v = 0; v < 3; ++v) {
-                double t = -1.0;
-                if (bd.n_fixed_jobs > 0) {
-                    set_tuning(pers[v], prev_tile);
+                if (bd.n_fixed_jobs > 0 && !(v > 0 && bd.fixed_wide)) {
+                    set_tuning(bd.fixed_wide ? prev_per : pers[v], prev_tile);
                     BatchDev b = bd;
                     b.inst = d_inst + 2L * n;
                     if (max_jobs > 0 && b.n_fixed_jobs > max_jobs) b.n_fixed_jobs = (int)max_jobs;
                     t = time_launch([&] { check(launch_batch_fixed(b, mode, stream), "fixed velocities"); });
-                    if (t < tbest) {
+                    if (t < tbest && !bd.fixed_wide) {
                         tbest = t;
                         best_per = pers[v];
                     }
@@ -607,7 +619,7 @@ struct sb_batch {
                 if (timings) timings[v] = t;
             }
             tbest = 1e300;
-            double t = -1.0;
+            t = -1.0;
             for (int v = 0; v < 3; ++v) {
                 if (targets && !(v > 0 && bd.targets_few)) {
                     set_tuning(best_per, bd.targets_few ? prev_tile : tiles[v]);
@@ -757,6 +769,8 @@ int sb_batch_get_tuning(const sb_batch* b, int* fixed_per, int* targets_tile) {
     *targets_tile = b->bd.targets_tile;
     return 0;
 }
+
+int sb_debug_batch_fixed_wide(const sb_batch* b) { return b ? b->bd.fixed_wide : -1; }
 
 int sb_debug_batch_targets_few(const sb_batch* b) { return b ? b->bd.targets_few : -1; }
 

@@ -129,8 +129,9 @@ struct McBuffers {
     int tmap_span = 0;  // span points per wave of the map (0: flat order)
 };
 
-// Control points per job of the batched fixed velocities (kb_fixed).
+// Control points per job of the batched fixed velocities (kb_fixed, kb_fixed_wide).
 constexpr int FIXED_JOB_TARGETS = 16;
+constexpr int FIXED_WIDE_TARGETS = 64;
 
 // Scratch of the two-pass few-target sum (k_terms + k_fold_terms): one chunk
 // of per-pair terms [3][n_targets][row] and the running sums [3][n_targets].
@@ -220,12 +221,13 @@ struct BatchDev {
     long blocks[BK_KINDS] = {};   // total flat blocks per kind
     int max_threads = 64;         // one-workgroup kernels: max over instances of N rounded to 64
     size_t solve_shm = 0;         // bytes of shared memory for the batched solve
-    const int2* fixed_jobs = nullptr;   // (instance, 64-target block), longest first
+    const int2* fixed_jobs = nullptr;   // (instance, 16- or 64-target block), longest first
     int n_fixed_jobs = 0;
     const int2* target_jobs = nullptr;  // (instance, 256-target block) of the free-wake self-induction
     int n_target_jobs = 0;
     unsigned* counters = nullptr;       // device [2] job-queue heads, zero between launches
-    int fixed_grid = 0, target_grid = 0;  // persistent workgroups
+    int fixed_grid = 0, fixed_wide_grid = 0, target_grid = 0;  // persistent workgroups
+    int fixed_wide = 0;           // 1 for kb_fixed_wide (batch_fixed_wide), its jobs 64 targets
     int fixed_per = 3;            // kb_fixed: fours of panels per compute wave per block (1, 2, 3)
     int targets_tile = 256;       // kb_targets: panel records per LDS tile (64, 128, 256)
     int cus = 0;                  // compute units of the batch's device
@@ -253,6 +255,9 @@ hipError_t launch_batch_factors(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_solve(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_velocity_copy(const BatchDev& b, hipStream_t st);
 hipError_t launch_batch_self_induction(const BatchDev& b, int mode, hipStream_t st);
+// Whether a batch's fixed velocities take kb_fixed_wide: the panels of the longest job, and
+// the panels of all jobs of FIXED_JOB_TARGETS and of FIXED_WIDE_TARGETS control points.
+bool batch_fixed_wide(int mode, int sym, int cus, double longest, double work, double work_wide);
 // Whether a batch of n_jobs target jobs with `panels` panels each on average takes
 // kb_targets_few (16 wake points per workgroup).
 bool batch_targets_few(int mode, int sym, int cus, long n_jobs, double panels);
@@ -274,9 +279,8 @@ size_t batch_linearized_shared(const int* ns, int n, int variant);
 hipError_t launch_batch_linearized(const BatchDev& b, int variant, size_t shm, int as_start, hipStream_t st);
 // Singular-pivot flags of every instance into flags[n] (device), cleared in the instances.
 hipError_t launch_batch_take_singular(const BatchDev& b, double* flags, hipStream_t st);
-// Resident workgroups of the persistent pair-sum kernels (0 fixed, 1 self-induction).
-// Resident workgroups of kb_fixed (which 0; variant = panels per wave) or
-// kb_targets (which 1; variant = tile length).
+// Resident workgroups of kb_fixed (which 0; variant = fours of panels per wave),
+// kb_targets (which 1; variant = tile length) or kb_fixed_wide (which 2).
 int batch_resident_groups(int which, int mode, int sym, int variant, int stage_near);
 
 }  // namespace sb

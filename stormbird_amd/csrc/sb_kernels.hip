@@ -3055,10 +3055,10 @@ __device__ inline double ordered_block_sum(const Inst& d, V3 x, int wt, int pb, 
 
 // Fixed velocities of many instances (frozen_wake.rs:189-261).  Job = one
 // instance's FX_TARGETS control points over its panels of rows >= 1.  Jobs are
-// taken longest first from a queue by persistent workgroups (96 polar instances, the
-// largest 372 strips x 1,000 rows: step 18.8 -> 9.6 ms against jobs of 64 control
-// points with a wave-uniform panel; 400 instances of up to 600 rows, where the queue
-// evens out either way: 22.1 -> 20.9).
+// taken longest first from a queue by persistent workgroups.  A job is one instance's
+// whole wake in order, so that the longest bounds the launch while the others don't fill
+// the GPU: there jobs of 16 control points serve where 64 (kb_fixed_wide) run long (96
+// polar instances, the largest 372 strips x 1,000 rows, EXACT: kernel 17.4 -> 5.4 ms).
 // PER x 4 panels per compute wave per block (PER 1, 2 or 3; the autotuner picks it).
 template <int MODE, int SYM, int PER>
 __global__ __launch_bounds__(FX_WAVES* WAVE) __attribute__((amdgpu_waves_per_eu(4))) void kb_fixed(
@@ -3078,6 +3078,126 @@ __global__ __launch_bounds__(FX_WAVES* WAVE) __attribute__((amdgpu_waves_per_eu(
                                                              d.N * d.nz_rows, T);
         if (threadIdx.x >= FX_COMPUTE * WAVE && lane < 3 * FX_TARGETS && t < d.N)
             d.fixed[3 * t + lane / FX_TARGETS] = acc;
+    }
+}
+
+// The same in jobs of 64 control points, a target per lane: the waves' panels are
+// wave-uniform, so that the records come by scalar loads and (without a symmetry plane)
+// three far evaluations run interleaved, and a pair costs less; but a job is four times as
+// long.  For batches whose work fills the GPU in such jobs (batch_fixed_wide).  Fifteen
+// compute waves evaluate PER consecutive panels each into one half of a double-buffered
+// LDS term array while the last wave adds the previous block's terms in ascending panel
+// order, one barrier per block.  Three panels per wave (2: 63.5 ms against 57.8 at 512
+// polar instances, FAST; 1: 83), mirrored evaluations one (more spill: 200 instances, FAST,
+// 37 ms against 107).  The registers are all in use: a running panel index, or a fold
+// without the partial block, spills more with a symmetry plane (those 200: 49.7 ms).
+template <int MODE, int SYM>
+__global__ __launch_bounds__(FX_WAVES* WAVE) void kb_fixed_wide(const Inst* I, const int2* __restrict__ jobs, int n_jobs,
+                                                                unsigned* head) {
+    constexpr int PER = SYM ? 1 : 3;
+    constexpr int FX_BLOCK = FX_COMPUTE * PER;
+    constexpr int FOLD_CHUNK = FX_BLOCK / 5;  // the fold's loads run one chunk ahead of its adds
+    static_assert(FX_BLOCK % FOLD_CHUNK == 0, "the fold reads full blocks in chunks");
+    static_assert(FIXED_WIDE_TARGETS == WAVE, "a target per lane");
+    __shared__ double T[2][FX_BLOCK][3][WAVE];  // 46,080 B per panel per wave
+    __shared__ int slot;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int lane = threadIdx.x % WAVE;
+    for (;;) {
+        int j = next_job(head, &slot);
+        if (j >= n_jobs) break;
+        int2 jb = jobs[j];
+        const Inst d = I[jb.x];
+        int t = jb.y * WAVE + lane;
+        int tc = t < d.N ? t : d.N - 1;
+        V3 x = load3(d.geo + d.gl.ctrl + 3 * tc);
+        int wt = d.neglect_self ? d.wing_of[tc] : -1;
+        const long p_begin = d.N, p_end = (long)d.N * d.nz_rows;
+        const long nblk = p_end > p_begin ? (p_end - p_begin + FX_BLOCK - 1) / FX_BLOCK : 0;
+        double acc = 0.0;
+        if (wave < FX_COMPUTE) {
+            ScalarRecs recs = (ScalarRecs)d.rec;
+            const int pb = (int)p_begin, pe = (int)p_end;
+            const int mine = pb + wave * PER;  // first panel of this wave in block 0
+            PanelRec r[PER];
+            if (nblk > 0) {
+#pragma unroll
+                for (int q = 0; q < PER; ++q) r[q] = scalar_rec(recs, mine + q < pe ? mine + q : pe - 1);
+            }
+            for (int b = 0; b <= (int)nblk; ++b) {
+                if (b < (int)nblk) {
+                    const int buf = b & 1;
+                    const int k0 = mine + b * FX_BLOCK;
+                    V3 term[PER];
+                    if constexpr (SYM == 0) {
+                        // far-field terms of the panels, interleaved; then the
+                        // lanes that need the general evaluation
+                        bool ok[PER];
+#pragma unroll
+                        for (int q = 0; q < PER; ++q) ok[q] = far_fast<MODE>(r[q], x, term[q]);
+#pragma unroll
+                        for (int q = 0; q < PER; ++q)
+                            if (!ok[q]) term[q] = panel_unit<MODE>(d, r[q], k0 + q < pe ? k0 + q : pe - 1, x);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < PER; ++q)
+                            term[q] = pair_unit<MODE, SYM>(d, r[q], k0 + q < pe ? k0 + q : pe - 1, x);
+                    }
+#pragma unroll
+                    for (int q = 0; q < PER; ++q) {
+                        const int k = k0 + q;
+                        bool skip = k >= pe || r[q].strength == 0.0 ||
+                                    (d.neglect_self && d.wing_of[k % d.N] == wt);
+                        V3 u = skip ? V3{0.0, 0.0, 0.0} : term[q] * r[q].strength;
+                        const int kl = wave * PER + q;
+                        T[buf][kl][0][lane] = u.x;
+                        T[buf][kl][1][lane] = u.y;
+                        T[buf][kl][2][lane] = u.z;
+                    }
+                    // records of the next block, loaded across the barrier
+                    const int kn = k0 + FX_BLOCK;
+#pragma unroll
+                    for (int q = 0; q < PER; ++q) r[q] = scalar_rec(recs, kn + q < pe ? kn + q : pe - 1);
+                }
+                __syncthreads();
+            }
+        } else {
+            double ay = 0.0, az = 0.0;
+            for (long b = 0; b <= nblk; ++b) {
+                if (b > 0) {
+                    const int buf = (int)((b - 1) & 1);
+                    const long base = p_begin + (b - 1) * FX_BLOCK;
+                    const int cnt = (int)(p_end - base < FX_BLOCK ? p_end - base : FX_BLOCK);
+                    if (cnt == FX_BLOCK) {
+                        // a full block: loads issued a chunk ahead of the adds
+#pragma unroll
+                        for (int q0 = 0; q0 < FX_BLOCK; q0 += FOLD_CHUNK) {
+                            double vx[FOLD_CHUNK], vy[FOLD_CHUNK], vz[FOLD_CHUNK];
+#pragma unroll
+                            for (int i = 0; i < FOLD_CHUNK; ++i) {
+                                vx[i] = T[buf][q0 + i][0][lane];
+                                vy[i] = T[buf][q0 + i][1][lane];
+                                vz[i] = T[buf][q0 + i][2][lane];
+                            }
+#pragma unroll
+                            for (int i = 0; i < FOLD_CHUNK; ++i) {
+                                acc = acc + vx[i];
+                                ay = ay + vy[i];
+                                az = az + vz[i];
+                            }
+                        }
+                    } else {
+                        for (int q = 0; q < cnt; ++q) {
+                            acc = acc + T[buf][q][0][lane];
+                            ay = ay + T[buf][q][1][lane];
+                            az = az + T[buf][q][2][lane];
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+            if (t < d.N) store3(d.fixed + 3 * t, V3{acc, ay, az});
+        }
     }
 }
 
@@ -3862,9 +3982,34 @@ static void launch_kb_fixed_per(const BatchDev& b, hipStream_t st) {
     else launch_kb_fixed<MODE, SYM, 3>(b, st);
 }
 
+// Either kernel's time is that of its longest job or of its jobs shared out evenly,
+// whichever is longer, at a cost per panel of a job: 38 (64 targets) against 13.6 ns (16)
+// in FAST, 105 against 65 with a symmetry plane, 147 against 62.8 in EXACT with one, 55
+// against 15.5 without (measured on polar batches of 4 to 512 instances, each within 5 %).
+// In EXACT without symmetry the wide jobs' cost per pair is no lower, and they don't pay
+// anywhere (512 instances: 83.6 ms against 82.6; their kernel is not built).  Wide pays
+// where the work fills the GPU: FAST, 512 instances of up to 3,000 rows 57.7 ms against
+// 72.9, 400 of up to 600 rows 12.6 against 15.1, 200 of up to 1,000 rows (still bounded by
+// the longest) 13.4 against 10.3; with a symmetry plane these 200 38.0 against 50.5, 512 of
+// up to 1,500 rows 88.3 against 196, in EXACT 119 against 184.
+bool batch_fixed_wide(int mode, int sym, int cus, double longest, double work, double work_wide) {
+    if (mode == MODE_EXACT && !sym) return false;
+    const double cost = mode == MODE_EXACT ? 2.35 : sym ? 1.62 : 2.8;  // of a panel of a wide job, in narrow ones
+    return cost * fmax(longest, work_wide / cus) < fmax(longest, work / cus);
+}
+
+template <int MODE, int SYM>
+static void launch_kb_fixed_wide(const BatchDev& b, hipStream_t st) {
+    hipLaunchKernelGGL((kb_fixed_wide<MODE, SYM>), dim3(b.fixed_wide_grid), dim3(FX_WAVES * WAVE), 0, st, b.inst,
+                       b.fixed_jobs, b.n_fixed_jobs, b.counters);
+}
+
 hipError_t launch_batch_fixed(const BatchDev& b, int mode, hipStream_t st) {
     if (b.n_fixed_jobs <= 0) return hipSuccess;
-    if (mode == MODE_FAST) b.sym ? launch_kb_fixed_per<MODE_FAST, 1>(b, st) : launch_kb_fixed_per<MODE_FAST, 0>(b, st);
+    if (b.fixed_wide) {
+        if (mode == MODE_FAST) b.sym ? launch_kb_fixed_wide<MODE_FAST, 1>(b, st) : launch_kb_fixed_wide<MODE_FAST, 0>(b, st);
+        else launch_kb_fixed_wide<MODE_EXACT, 1>(b, st);
+    } else if (mode == MODE_FAST) b.sym ? launch_kb_fixed_per<MODE_FAST, 1>(b, st) : launch_kb_fixed_per<MODE_FAST, 0>(b, st);
     else b.sym ? launch_kb_fixed_per<MODE_EXACT, 1>(b, st) : launch_kb_fixed_per<MODE_EXACT, 0>(b, st);
     hipLaunchKernelGGL(kb_zero_counters, dim3(1), dim3(64), 0, st, b.counters);
     return hipGetLastError();
@@ -4009,6 +4154,12 @@ static int target_groups_staged(int tile, int stage_near) {
 }
 
 int batch_resident_groups(int which, int mode, int sym, int variant, int stage_near) {
+    if (which == 2) {  // EXACT takes the wide jobs with a symmetry plane only
+        const int th = FX_WAVES * WAVE;
+        if (mode == MODE_FAST && !sym) return resident_groups(kb_fixed_wide<MODE_FAST, 0>, th);
+        return mode == MODE_FAST ? resident_groups(kb_fixed_wide<MODE_FAST, 1>, th)
+                                 : resident_groups(kb_fixed_wide<MODE_EXACT, 1>, th);
+    }
     if (which == 0) {
         if (mode == MODE_FAST) return sym ? fixed_groups<MODE_FAST, 1>(variant) : fixed_groups<MODE_FAST, 0>(variant);
         return sym ? fixed_groups<MODE_EXACT, 1>(variant) : fixed_groups<MODE_EXACT, 0>(variant);

@@ -315,6 +315,60 @@ def test_residual_warm_start_with_a_zero_network_is_the_default_guess():
     assert b.batch.last_fallbacks() == 0
 
 
+def wide_route(batch):
+    """1 when the batch's last fixed velocities ran in jobs of 64 control points, 0 in jobs of 16."""
+    import ctypes
+
+    L = sb.lib()
+    L.sb_debug_batch_fixed_wide.argtypes = [ctypes.c_void_p]
+    return L.sb_debug_batch_fixed_wide(batch._h)
+
+
+@pytest.mark.parametrize("neglect", [False, True])
+@pytest.mark.parametrize("mode,symmetry", [(sb.MODE_FAST, None), (sb.MODE_FAST, "Z"), (sb.MODE_EXACT, "Z"),
+                                           (sb.MODE_EXACT, None)])
+def test_fixed_velocity_jobs_of_64_control_points(mode, symmetry, neglect):
+    """Sixty copies of twelve instances fill the GPU in jobs of 64 control points, which FAST arithmetic and
+    symmetry planes then take.  Control points below, at and above a job's
+    64, wakes from 2 rows (fewer panels than a block) up: the bits of the instances alone and of one
+    copy of each (jobs of 16), and the tuner times the one kernel once and leaves its parameter."""
+    import json
+
+    setups = []
+    for sails, strips, rows in [(1, 1, 2), (1, 15, 3), (1, 16, 9), (1, 17, 6), (1, 63, 8), (1, 64, 8), (1, 65, 3),
+                                (3, 5, 12), (2, 17, 8), (4, 4, 2), (1, 64, 9), (2, 32, 9)]:
+        js, case = S.four_sail_free_wake(nr_panels=rows, nr_strips=strips, ratio=0.0)
+        d = json.loads(js)
+        d["line_force_model"]["wing_builders"] = d["line_force_model"]["wing_builders"][:sails]
+        wake = d["simulation_settings"]["Dynamic"]["wake"]
+        if neglect:
+            wake["neglect_self_induced_velocities"] = True
+        if symmetry:
+            wake["symmetry_condition"] = symmetry
+        setups.append(json.dumps(d))
+    n = len(setups)
+    many, once = sb.Batch(setups * 60, mode=mode), sb.Batch(setups, mode=mode)
+    alone = [sb.Simulation(js, mode=mode) for js in setups]
+    parts = [S.uniform_freestream(a.nr_freestream_points(), case["velocity"]) for a in alone]
+    for k in range(13):
+        rm = many.do_step(times=0.2 * k, time_steps=0.2, freestream_velocity=np.concatenate(parts * 60))
+        ro = once.do_step(times=0.2 * k, time_steps=0.2, freestream_velocity=np.concatenate(parts))
+        assert wide_route(once) == 0
+        if k > 3:
+            assert wide_route(many) == (1 if mode == sb.MODE_FAST or symmetry else 0)
+        for i, a in enumerate(alone):
+            ra = a.do_step(time=0.2 * k, time_step=0.2, freestream_velocity=parts[i])
+            compare_results(ro[i], ra, exact=True, where=f"step {k} instance {i}")
+            for j in (0, 23, 59):
+                compare_results(rm[j * n + i], ra, exact=True, where=f"step {k} instance {i}, copy {j}")
+    many.set_tuning(2, 256)
+    _, choice, t = many.autotune(None)
+    if wide_route(many):
+        assert choice[0] == 2 and t[0] == t[1] == t[2] > 0.0
+    else:
+        assert len(set(t[:3])) > 1 and np.all(t[:3] > 0.0)
+
+
 def few_route(batch):
     """1 when the batch's last self-induction took the kernel for few wake points, else 0."""
     import ctypes
