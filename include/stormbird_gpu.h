@@ -272,6 +272,9 @@ int sb_debug_gauss_blocked_device(const double* A, const double* b, size_t n, do
  * out[0] = (((s0 + terms[0]) + terms[1]) + ...), rounded after every addition
  * (s0 not -0).  Returns 0, -1 on bad arguments, -2 on a device error. */
 int sb_debug_ordered_sum_device(const double* terms, size_t n, double s0, double* out);
+/* The rule that gives n_targets points with n_panels panels the kernel with 16 points per
+ * workgroup (1) or 256 (0) on a device of `cus` compute units. */
+int sb_debug_targets_few(int mode, int symmetric, int cus, long n_targets, long n_panels, int self_induction);
 
 /* ---- Batched simulations ------------------------------------------------
  * Many independent simulations (each built from its own setup string, with

@@ -178,6 +178,8 @@ hipError_t launch_velocity_copy(const Inst& d, hipStream_t st);
 hipError_t launch_copy3(const double* src, double* dst, long n, hipStream_t st);
 // dst[0, count) = src[0, count); src may be pinned host memory
 hipError_t launch_copy_doubles(const double* src, double* dst, long count, hipStream_t st);
+// Whether n_targets points take k_targets_few (16 per workgroup) rather than k_targets.
+bool targets_few(int mode, int sym, int cus, long n_targets, long n_panels, int self_induction);
 hipError_t launch_self_induction(const Inst& d, int mode, McBuffers* mc, hipStream_t st);
 // Induced velocity at `targets` from panels [0, n_panels): out (+)= sum.
 hipError_t launch_targets(const Inst& d, const double* targets, long n_targets, long n_panels, int mode, double* out,

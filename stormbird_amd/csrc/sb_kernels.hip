@@ -15,8 +15,6 @@
 // a refined reciprocal square root instead.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-
 #include "sb_device.h"
 #include "sb_wind.h"
 #include "sb_mlp.h"
@@ -3767,16 +3765,32 @@ hipError_t launch_velocity_copy(const Inst& d, hipStream_t st) {
     return hipGetLastError();
 }
 
-static long cu_count() {
-    static std::atomic<long> cached{0};
-    long c = cached.load(std::memory_order_relaxed);
-    if (c == 0) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
-            c = v;
-        cached.store(c, std::memory_order_relaxed);
-    }
-    return c;
+// Compute units of the current device (0 where it can't be asked).
+static int cu_count() {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    return v;
+}
+
+// As batch_targets_few, for one simulation's points (kernel ms few / 256-point, at
+// workgroups of 256 on 256 CUs; a free wake's self-induction):
+//   EXACT           379: 57.2 / 70.6, 450: 87.6 / 91.8 per step    -> 24/16 (shared with FAST)
+//   EXACT, symmetry 379: 126 / 147                                 -> 24/16
+//   FAST            379: 46.1 / 50.4, 450: 71.1 / 66.2 per step    -> 24/16
+//   FAST, symmetry  379, 4,000 panels: 3.74 / 4.89, 8,000: 6.86 / 6.81, 32,000: 28.3 / 21.7,
+//                   94,000: 116 / 106; 321, 80,000: 82.6 / 83.4    -> 24/16, from 8,000 panels on 19/16
+//                   points far from the panels: 384, 96,000: 78.4 / 94.9 -> 24/16
+// Few panels: the 256-point kernel's time goes with the panels alone, the few-point
+// kernel's with the points in whole blocks of 180 panels.  A call of induced velocities at
+// 98,304 points: 20 panels 0.50 ms / 0.37, 40: 0.495 / 0.443, 60: 0.485 / 0.524; at 40,000: 20
+// panels 0.218 / 0.179, 40: 0.218 / 0.231; at 20,000: 20 panels 0.141 / 0.141, with a symmetry
+// plane the same lines.  Self-induction in the first steps, where pairs are near: 72,000
+// points, 32 panels 0.095 / 0.106, with a symmetry plane 0.172 / 0.147, 40 panels 0.175 / 0.179.
+bool targets_few(int mode, int sym, int cus, long n_targets, long n_panels, int self_induction) {
+    const long jobs = (n_targets + 255) / 256, limit = mode == MODE_FAST && sym && self_induction && n_panels >= 8000 ? 19 : 24;
+    const long points = self_induction ? (sym ? 2000 : 3000) : 1000;  // per panel
+    return mode != MODE_FP32_KAHAN && 16 * jobs <= limit * cus && (n_panels >= 64 || n_targets <= points * n_panels);
 }
 
 template <int MODE, int SYM, bool NB>
@@ -3819,10 +3833,7 @@ static hipError_t launch_targets_t(const Inst& d, const double* targets, long n_
                                n_targets, out, add, pl);
     } else {
         if constexpr (MODE != MODE_FP32_KAHAN) {
-            // up to 1.5 workgroups of 256 per CU (there the two take the same time within 7 %
-            // either way, measured at 450 of them: EXACT 87.6 ms against 91.8, FAST 71.1
-            // against 66.2; at 176: 11.8 against 25.5 and 9.7 against 18.9)
-            if (!tmap && 2 * n_jobs <= 3 * cu_count()) {
+            if (!tmap && targets_few(MODE, SYM, cu_count(), n_targets, n_panels, add)) {
                 hipLaunchKernelGGL((k_targets_few<MODE, SYM>), dim3(blocks_for(n_targets, FX_TARGETS)),
                                    dim3(FX_WAVES * WAVE), 0, st, d, targets, n_targets, n_panels, out, add);
                 return hipGetLastError();

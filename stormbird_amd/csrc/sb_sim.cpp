@@ -471,6 +471,10 @@ int sb_debug_ordered_sum_device(const double* terms, size_t n, double s0, double
     return rc;
 }
 
+int sb_debug_targets_few(int mode, int symmetric, int cus, long n_targets, long n_panels, int self_induction) {
+    return targets_few(mode, symmetric, cus, n_targets, n_panels, self_induction);
+}
+
 int sb_debug_libm_host(int fn, const double* x, const double* y, double* out, size_t n) {
     if (!x || !out || (fn == 4 && !y)) return -1;
     for (size_t i = 0; i < n; ++i) {

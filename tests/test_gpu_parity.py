@@ -496,3 +496,29 @@ def test_target_tiling_leaves_results_unchanged(oracle):
         step_both(gpu, orc, fs, 12, case["time_step"], wake_check_every=4)
     with pytest.raises(RuntimeError):
         sb.Simulation(js).target_tiling = 3
+
+
+@pytest.mark.parametrize("symmetry", [None, "Z"])
+@pytest.mark.parametrize("mode", [sb.MODE_EXACT, sb.MODE_FAST])
+def test_induced_velocities_on_both_sides_of_the_kernel_rules(mode, symmetry):
+    """The same points in one call and in parts give the same bits: 40,000 points of 20 panels (the
+    256-point kernel) and in tens of thousands (16 points per workgroup); 100,000 points of 180 panels
+    (the 256-point kernel, above its bound) and in halves; and parts of 2,000 (a wave per point)."""
+    import json
+
+    rng = np.random.default_rng(17)
+    for strips, rows, n, part in ((20, 1, 40_000, 10_000), (20, 9, 100_000, 50_000)):
+        js, case = S.four_sail_free_wake(nr_panels=rows, nr_strips=strips, ratio=0.0)
+        d = json.loads(js)
+        d["line_force_model"]["wing_builders"] = d["line_force_model"]["wing_builders"][:1]
+        if symmetry:
+            d["simulation_settings"]["Dynamic"]["wake"]["symmetry_condition"] = symmetry
+        sim = sb.Simulation(json.dumps(d), mode=mode)
+        fs = S.uniform_freestream(sim.nr_freestream_points(), case["velocity"])
+        for k in range(rows + 2):
+            sim.do_step(time=0.2 * k, time_step=0.2, freestream_velocity=fs)
+        points = rng.uniform(-40.0, 40.0, (n, 3))
+        whole = sim.induced_velocities(points)
+        assert np.all(np.isfinite(whole)) and np.any(whole)
+        assert same(np.concatenate([sim.induced_velocities(points[a:a + part]) for a in range(0, n, part)]), whole)
+        assert same(sim.induced_velocities(points[:2000]), whole[:2000])

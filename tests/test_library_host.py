@@ -204,3 +204,27 @@ def test_setup_check_applies_the_create_time_limits():
     assert ok["nr_ctrl_points"] == 1024
     with pytest.raises(ValueError, match="1024"):
         sb.setup_info(S.rectangular_wing(nr_strips=1025, nr_panels=2))
+
+
+@pytest.mark.parametrize("mode,symmetric,most,long", [(0, 0, 384, 384), (0, 1, 384, 384), (1, 0, 384, 384),
+                                                      (1, 1, 384, 304), (2, 0, 0, 0), (2, 1, 0, 0)])
+def test_rule_for_the_few_point_kernel(mode, symmetric, most, long):
+    """On 256 CUs, `most` workgroups of 256 points (none in FP32-Kahan, which the kernel does not have),
+    `long` of them in a self-induction from 8,000 panels on; with few panels the points a panel pays for: 1,000 in a call of induced velocities, 2,000 or 3,000 in
+    the self-induction, any from 64 panels on."""
+    rule = sb.lib().sb_debug_targets_few
+    rule.argtypes = [ctypes.c_int] * 3 + [ctypes.c_long] * 2 + [ctypes.c_int]
+
+    def few(points, panels, own):
+        return rule(mode, symmetric, 256, points, panels, own)
+
+    for own, per_panel in ((0, 1000), (1, 2000 if symmetric else 3000)):
+        assert few(256 * most, 64, own) == (most > 0)
+        assert few(256 * most + 1, 7999, own) == 0
+        assert few(256 * (long if own else most), 8000, own) == (most > 0)
+        assert few(256 * (long if own else most) + 1, 8000, own) == 0
+        for panels in (1, 20, 24):
+            assert few(per_panel * panels, panels, own) == (most > 0)
+            assert few(per_panel * panels + 1, panels, own) == 0
+        assert few(65 * 1000, 63, own) == (most > 0 and own)
+    assert rule(mode, symmetric, 0, 300, 100, 0) == 0  # a device that can't be asked
