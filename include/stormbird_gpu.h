@@ -275,6 +275,9 @@ int sb_debug_ordered_sum_device(const double* terms, size_t n, double s0, double
 /* The rule that gives n_targets points with n_panels panels the kernel with 16 points per
  * workgroup (1) or 256 (0) on a device of `cus` compute units. */
 int sb_debug_targets_few(int mode, int symmetric, int cus, long n_targets, long n_panels, int self_induction);
+/* The same rule of a batch's self-induction: n_jobs workgroups of 256 points, `panels`
+ * panels each on average. */
+int sb_debug_batch_few_rule(int mode, int symmetric, int cus, long n_jobs, double panels);
 
 /* ---- Batched simulations ------------------------------------------------
  * Many independent simulations (each built from its own setup string, with

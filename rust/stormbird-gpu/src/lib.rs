@@ -140,6 +140,7 @@ pub mod ffi {
         pub fn sb_debug_gauss_device(a: *const f64, b: *const f64, n: usize, x: *mut f64, variant: c_int) -> c_int;
         pub fn sb_debug_gauss_blocked_device(a: *const f64, b: *const f64, n: usize, x: *mut f64) -> c_int;
         pub fn sb_debug_targets_few(mode: c_int, symmetric: c_int, cus: c_int, n_targets: c_long, n_panels: c_long, self_induction: c_int) -> c_int;
+        pub fn sb_debug_batch_few_rule(mode: c_int, symmetric: c_int, cus: c_int, n_jobs: c_long, panels: f64) -> c_int;
         pub fn sb_debug_ordered_sum_device(terms: *const f64, n: usize, s0: f64, out: *mut f64) -> c_int;
         pub fn sb_batch_create(setup_jsons: *const *const c_char, n: c_long, device: c_int, mode: c_int) -> *mut sb_batch;
         pub fn sb_batch_destroy(b: *mut sb_batch);

@@ -4084,18 +4084,26 @@ hipError_t launch_batch_velocity_copy(const BatchDev& b, hipStream_t st) {
 // The few-point kernel's time goes with the jobs, the 256-point kernel's is that of its
 // longest workgroups while every CU has at most one or two, so up to a number of jobs per
 // CU the first is faster (kernel ms few / 256-point, tile 256, at workgroups of 256 on 256
-// CUs):
-//   EXACT           624: 15.2 / 16.6, 702: 17.1 / 16.9, 758: 113 / 116        -> 3 per CU
-//   EXACT, symmetry 266: 11.1 / 11.7, 297: 8.9 / 9.6, 312: 25.1 / 23.4, 624: 49.8 / 32.5 -> 19/16
-//   FAST            312: 6.65 / 7.92, 379: 47.2 / 50.2, 390 extrapolated: 8.3 / 7.9 -> 24/16
-//   FAST, symmetry  156: 13.4 / 15.3, 161: 31.1 / 34.5, 204: 15.1 / 13.3, 312: 26.7 / 16.2 -> 11/16
-// (FAST gains more from the 256-point kernel's wave-uniform panel, and so does the mirrored
-// evaluation.)  And it works through whole blocks of 180 panels, so that few panels (the
+// CUs, four-sail wakes):
+//   EXACT           624: 15.2 / 16.6, 702: 17.1 / 16.9, 758: 113 / 116               -> 3 per CU
+//   FAST            312: 6.65 / 7.92, 379: 47.2 / 50.2, 390 extrapolated: 8.3 / 7.9  -> 24/16
+// With a symmetry plane the few-point kernel spills, and the line depends on the panels (the
+// 256-point kernel waits on its tiles while they are few):
+//   EXACT           768 panels: 468: 1.78 / 1.90, 624: 2.37 / 2.14                   -> 32/16
+//                   2,080: 379: 3.13 / 3.61; 2,688: 312: 3.3 / 4.3, 468: 4.97 / 4.45 -> 24/16
+//                   10,000 and more: 266: 11.1 / 11.7, 297: 8.9 / 9.6, 312: 13.1 / 12.9, 624: 49.8 / 32.5 -> 19/16
+//   FAST            768 panels: 312: 1.28 / 1.56, 1,408: 312: 1.97 / 2.38            -> 22/16
+//                   2,688: 234: 2.71 / 3.30, 312: 3.60 / 3.31                        -> 17/16
+//                   5,248: 234: 5.36 / 5.31                                          -> 13/16
+//                   10,000 and more: 156: 13.4 / 15.3, 161: 31.1 / 34.5, 204: 15.1 / 13.3, 312: 26.7 / 16.2 -> 10/16
+// And the few-point kernel works through whole blocks of 180 panels, so that fewer (the
 // first steps after the start) don't pay with many points:
 //   EXACT           145,000 points: 40 panels 0.210 / 0.145, 56: 0.205 / 0.197, 72: 0.206 / 0.225; 72,000: 40: 0.109 / 0.132
 //   EXACT, symmetry 72,000 points: 40 panels 0.33 / 0.18, 72: 0.33 / 0.29; 63,000: 100: 0.30 / 0.35
 bool batch_targets_few(int mode, int sym, int cus, long n_jobs, double panels) {
-    const long limit = mode == MODE_EXACT ? (sym ? 19 : 48) : (sym ? 11 : 24);
+    const bool exact = mode == MODE_EXACT;
+    long limit = exact ? 48 : 24;  // sixteenths per CU
+    if (sym) limit = panels < 1500 ? (exact ? 32 : 22) : panels < 3000 ? (exact ? 24 : 17) : exact ? 19 : panels < 6000 ? 13 : 10;
     return 16 * n_jobs <= limit * cus && 256.0 * (double)n_jobs <= (sym ? 850.0 : 2500.0) * panels;
 }
 

@@ -475,6 +475,10 @@ int sb_debug_targets_few(int mode, int symmetric, int cus, long n_targets, long 
     return targets_few(mode, symmetric, cus, n_targets, n_panels, self_induction);
 }
 
+int sb_debug_batch_few_rule(int mode, int symmetric, int cus, long n_jobs, double panels) {
+    return batch_targets_few(mode, symmetric, cus, n_jobs, panels);
+}
+
 int sb_debug_libm_host(int fn, const double* x, const double* y, double* out, size_t n) {
     if (!x || !out || (fn == 4 && !y)) return -1;
     for (size_t i = 0; i < n; ++i) {

@@ -228,3 +228,22 @@ def test_rule_for_the_few_point_kernel(mode, symmetric, most, long):
             assert few(per_panel * panels + 1, panels, own) == 0
         assert few(65 * 1000, 63, own) == (most > 0 and own)
     assert rule(mode, symmetric, 0, 300, 100, 0) == 0  # a device that can't be asked
+
+
+@pytest.mark.parametrize("mode,symmetric,lines", [
+    (0, 0, [(100, 768), (10 ** 6, 768)]), (1, 0, [(100, 384), (10 ** 6, 384)]),
+    (0, 1, [(768, 512), (1499, 512), (1500, 384), (2999, 384), (3000, 304), (10 ** 6, 304)]),
+    (1, 1, [(768, 352), (1499, 352), (1500, 272), (2999, 272), (3000, 208), (5999, 208), (6000, 160), (10 ** 6, 160)]),
+])
+def test_rule_for_the_few_point_kernel_of_a_batch(mode, symmetric, lines):
+    """On 256 CUs: the most workgroups of 256 points at an average of panels, and the points that a panel
+    pays for while there are few (2,500, mirrored 850)."""
+    rule = sb.lib().sb_debug_batch_few_rule
+    rule.argtypes = [ctypes.c_int] * 3 + [ctypes.c_long, ctypes.c_double]
+    for panels, most in lines:
+        assert rule(mode, symmetric, 256, most, float(panels)) == 1
+        assert rule(mode, symmetric, 256, most + 1, float(panels)) == 0
+    per_panel = 850 if symmetric else 2500
+    for jobs in (50, 100):
+        assert rule(mode, symmetric, 256, jobs, 256.0 * jobs / per_panel) == 1
+        assert rule(mode, symmetric, 256, jobs, 256.0 * jobs / per_panel - 0.01) == 0
