@@ -259,13 +259,14 @@ int sb_debug_libm_host(int fn, const double* x, const double* y, double* out, si
 int sb_debug_linearized_in_shared_memory(long n_strips);
 /* The one-workgroup Gaussian elimination with partial pivoting that the
  * Linearized solve runs (stormath matrix/linalg.rs:41-104), on a given system:
- * A row-major n x n, b [n], x [n]; variant 1 (256 threads, n <= 64), 2 (256,
- * n <= 127), 3 (256, n <= 128) or 4 (512, n <= 139).  Returns 0, k + 1 when the pivot of step k is
+ * A row-major n x n, b [n], x [n]; variant 1 (one 64-row slice, 256 threads, n <= 64),
+ * 2 or 3 (two slices, 512 threads; one kernel, taken up to n = 127 and 128) or 4 (three
+ * slices, 512 threads, n <= 139).  Returns 0, k + 1 when the pivot of step k is
  * below 1e-12 in magnitude (where linalg.rs:67-71 returns its error; x is then
  * zero), -1 when n does not fit the variant, -2 on a device error. */
 int sb_debug_gauss_device(const double* A, const double* b, size_t n, double* x, int variant);
 /* The same elimination in the blocked form the Linearized solve takes for larger
- * systems (16-column panels, trailing updates, one-wave back substitution), the
+ * systems (16-column panels, trailing updates, back substitution in one workgroup), the
  * matrix in global memory: n <= 1024.  Returns as sb_debug_gauss_device. */
 int sb_debug_gauss_blocked_device(const double* A, const double* b, size_t n, double* x);
 /* The ordered sum that the fixed velocities' fold runs on one wave, on given terms:

@@ -272,8 +272,8 @@ hipError_t launch_batch_warm_start(const BatchDev& b, sb_mlp* mlp, int apply, hi
 // solver's first evaluation (after the factors, before the solve).
 hipError_t launch_batch_warm_judge(const BatchDev& b, hipStream_t st);
 // Quasi-steady batches: horseshoe factors of every instance, and the
-// one-workgroup Linearized solve per instance (variant 1: N <= 128, 2: larger;
-// 0 when max_n needs the blocked form, which batches do not run).
+// one-workgroup Linearized solve per instance (variant 1: N <= 64, 2: N <= 128, 3: what
+// shared memory holds; 0 when max_n needs the blocked form, which batches do not run).
 hipError_t launch_batch_horseshoe_factors(const BatchDev& b, hipStream_t st);
 int batch_linearized_variant(int max_n);
 // Shared memory of the variant for instances of ns[0..n) strips (0: one does not fit).

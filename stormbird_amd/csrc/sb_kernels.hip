@@ -1060,7 +1060,6 @@ __device__ inline double ordered_sum_wave(double s, const double (&p)[M]) {
     bool fine = lo12 == hi12 && hi12 != 0u && hi12 != 0x7ffu;  // |g| - reach < 0: its sign bit makes them differ
     fine = fine && d0 > -SMALL && d0 < SMALL && d1 > -SMALL && d1 < SMALL;
     fine = fine || (reach == 0.0 && gb == nb);  // adding zeros changes nothing
-    const unsigned long long good = __ballot(fine);
     // Lanes below j0 are done (leading lanes of zeros change nothing); sx is the exact
     // sum before lane j0, which is the first of its run or follows leading zeros.
     const unsigned long long some = __ballot(!(reach == 0.0));

@@ -246,9 +246,10 @@ def test_batch_rejects_mixed_and_warm_quasi():
 @pytest.mark.parametrize("symmetric", [False, True])
 def test_autotuner_and_every_variant_keep_results(tmp_path, symmetric):
     """The autotuner times the kernel variants on the batch's own state without changing
-    it; every variant (panels per wave of the fixed-velocity kernel, LDS tile length of the
-    self-induction kernel) gives the same bits; the choice is cached per device and shape
-    class in a JSON file and reused by a batch of the same shape."""
+    it; every variant (fours of panels per wave of the fixed-velocity kernel, LDS tile length of
+    the self-induction kernel, which this small wake does not reach:
+    test_every_self_induction_kernel_gives_the_same_bits) gives the same bits; the choice is
+    cached per device and shape class in a JSON file and reused by a batch of the same shape."""
     import json
 
     setups, cases = mixed_setups()

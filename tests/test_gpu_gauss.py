@@ -5,9 +5,9 @@ systems through sb_debug_gauss_device.
 The solution must equal the oracle's bit for bit: the same pivot choice (largest
 magnitude, the first of equal ones, a NaN at the pivot position kept), the same
 a - f * p updates and the same ascending-column back substitution.  Cases: random
-systems of every size class of the four register layouts (one to three 64-row
-slices of the pivot search, two to four rows and 12-20 columns per thread) and of the
-blocked form (16-column panels; partial and several panels, up to 1024 rows), systems with many equal
+systems of every size class of the one-workgroup form (panels of 8 columns factored in
+one wave's registers, one to three 64-row slices; the variants 2 and 3 are one kernel under two
+row limits) and of the blocked form (16-column panels; partial and several panels, up to 1024 rows), systems with many equal
 magnitudes (pivot ties), zero diagonals (row exchanges at every step), NaN and
 infinite entries, and singular systems, whose failing step must be the oracle's.
 """
@@ -29,7 +29,7 @@ def _p(a):
 
 
 def gpu_solve(A, b, variant):
-    """variant 1-4: the one-workgroup register layouts; "blocked": the global-memory form."""
+    """variant 1-4: the one-workgroup form; "blocked": the global-memory form."""
     L = sb.lib()
     A = np.ascontiguousarray(A, dtype=np.float64)
     b = np.ascontiguousarray(b, dtype=np.float64)

@@ -503,11 +503,12 @@ def test_target_tiling_leaves_results_unchanged(oracle):
 def test_induced_velocities_on_both_sides_of_the_kernel_rules(mode, symmetry):
     """The same points in one call and in parts give the same bits: 40,000 points of 20 panels (the
     256-point kernel) and in tens of thousands (16 points per workgroup); 100,000 points of 180 panels
-    (the 256-point kernel, above its bound) and in halves; and parts of 2,000 (a wave per point)."""
+    (the 256-point kernel, above its bound) and in halves; 300,000 (the balanced kernel) and in thirds
+    (the 256-point kernel); and parts of 2,000 (a wave per point)."""
     import json
 
     rng = np.random.default_rng(17)
-    for strips, rows, n, part in ((20, 1, 40_000, 10_000), (20, 9, 100_000, 50_000)):
+    for strips, rows, n, part in ((20, 1, 40_000, 10_000), (20, 9, 100_000, 50_000), (20, 9, 300_000, 100_000)):
         js, case = S.four_sail_free_wake(nr_panels=rows, nr_strips=strips, ratio=0.0)
         d = json.loads(js)
         d["line_force_model"]["wing_builders"] = d["line_force_model"]["wing_builders"][:1]

@@ -34,7 +34,7 @@ def test_noalloc_matches_allocating_entry():
     d_t = torch.from_numpy(targets).to("cuda")
     d_out = torch.full((6000, 3), float("nan"), dtype=torch.float64, device="cuda")
     for symmetry, mode in ((0, sb.MODE_EXACT), (3, sb.MODE_FAST)):
-        # first call: 4800 panels, 6000 targets (the 256-target block kernel); second call:
+        # first call: 4800 panels, 6000 targets (16 per workgroup); second call:
         # 1000 panels, 500 targets (the few-target kernel), reusing the scratch of the first
         for n_p, n_t in ((4800, 6000), (1000, 500)):
             print(f"noalloc: symmetry {symmetry} mode {mode} panels {n_p} targets {n_t}", flush=True)
