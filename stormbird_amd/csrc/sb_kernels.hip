@@ -1962,8 +1962,7 @@ SB_HD constexpr LinrLayout linr_layout(int N) {
     LinrLayout L{};
     L.ld = N | 1;
     L.pstride = (int)(N + 40 > 64 * LINR_PS ? linr_even(N + 40) : 64 * LINR_PS);
-    const long matrix = (long)(N + 1) * L.ld, induced = 3L * N;
-    L.G = linr_even(matrix > induced ? matrix : induced);
+    L.G = linr_even((long)(N + 1) * L.ld + 2);  // + 2: the induced velocities at N = 1
     L.R = L.G + linr_even(N + 8);
     L.prod = L.R + linr_even(N);
     L.src = L.prod + 2L * L.pstride + 16;
