@@ -2978,7 +2978,7 @@ __device__ inline int next_job(unsigned* head, int* slot) {
 // A sum over panels is a chain, so the parallel work is in the targets: 16 of them on a
 // whole CU serve where 64 or 256 per workgroup leave the chip with too few waves, or
 // with a few that run long.
-constexpr int FX_WAVES = 16;              // a job on a whole CU (8: 10.4 ms on the polar batch below, 4: 18.9)
+constexpr int FX_WAVES = 16;              // a job on a whole CU (step of the polar batch below 9.6 ms; with 8 waves 10.4, with 4 18.9)
 constexpr int FX_COMPUTE = FX_WAVES - 1;  // compute waves; the last wave folds
 constexpr int FX_TARGETS = FIXED_JOB_TARGETS;
 constexpr int FX_SUB = WAVE / FX_TARGETS; // panels side by side in a wave
