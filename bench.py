@@ -259,7 +259,7 @@ def batched_polar_sweep(n_inst=512, seed=2, steps=3, plain_steps=1, mode=0, mlp=
         "mode": {0: "exact", 1: "fast"}[mode],
         "iterations_mean": float(np.mean(iters)),
         "autotuner": {"fixed_per": tuning[0], "targets_tile": tuning[1],
-                      "fixed_ms_per_panels_per_wave_1_2_3": [float(x) for x in tune_ms[:3]]},
+                      "fixed_ms_per_variant_1_2_3": [float(x) for x in tune_ms[:3]]},
         "warm_start": warm,
     }
 
