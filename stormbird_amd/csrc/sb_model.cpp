@@ -315,7 +315,6 @@ static void add_wing(LineModel& m, const Node* wb, int default_sections) {
     m.wing_end.push_back(start + count);
     m.foils.push_back(foil);
     m.wing_angles.push_back(0.0);
-    m.update_global();
 }
 
 static LineModel parse_line_model(const Node* o) {  // builder/mod.rs:79-113
@@ -331,6 +330,11 @@ static LineModel parse_line_model(const Node* o) {  // builder/mod.rs:79-113
     if (!wbs || wbs->t != Node::Arr || wbs->items.empty())
         throw std::runtime_error("LineForceModelBuilder: wing_builders must be a non-empty list");
     for (auto& wb : wbs->items) add_wing(m, wb.get(), nsec);
+    // A wing of zero length has no strips.  Its one span point lies at the end of the strip
+    // before it and takes the values of the strip behind it, so it needs both.
+    for (int w = 0; w < m.nw(); ++w)
+        if (m.wing_start[w] == m.wing_end[w] && (m.wing_start[w] == 0 || m.wing_start[w] == m.n()))
+            throw std::runtime_error("wing " + std::to_string(w) + " has no strips (zero length) and no wing with strips on both sides");
     const Node* p;
     if (const Node* v = o->find("circulation_correction"))
         if (variant(v, &p, "CirculationCorrectionBuilder") != "None")

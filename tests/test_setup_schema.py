@@ -224,3 +224,34 @@ def test_valid_setups_outside_this_library_name_the_feature(model, msg):
     d = base()
     d["line_force_model"]["circulation_correction"] = {"Prescribed": {}}
     rejects(d, "circulation correction")
+
+
+def test_wings_without_strips_at_either_end_are_rejected():
+    """A wing of zero length between others is taken (no strips, one span point); first or last there is no
+    strip that its span point could take its values from.  In a process of its own: reading them
+    anyway ends it."""
+    import subprocess
+    import sys
+
+    code = """
+import json
+import stormbird_amd as sb
+from stormbird_amd import setups as S
+for dynamic in (False, True):
+    for at in (0, 1, 2):
+        d = json.loads(S.wing_sails_quasi_steady(nr_strips=4))
+        if dynamic:
+            d["simulation_settings"] = S.dynamic_settings(nr_panels=5)
+        w = d["line_force_model"]["wing_builders"][at]
+        w["section_points"][1] = dict(w["section_points"][0])
+        try:
+            i = sb.setup_info(json.dumps(d))
+            print(at, i["nr_ctrl_points"], i["nr_wings"], i["nr_span_points"])
+        except ValueError as e:
+            print(at, e)
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    want = ["0 wing 0 has no strips (zero length) and no wing with strips on both sides", "1 8 3 11",
+            "2 wing 2 has no strips (zero length) and no wing with strips on both sides"]
+    assert r.returncode == 0 and r.stdout.splitlines() == want * 2, (r.returncode, r.stdout, r.stderr[-500:])
